@@ -162,8 +162,8 @@ int trhip_gemm_q_typed(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int6
 
 /* ActQuantGemmer.GemmActQuant (tensor/matmul.go:59-61, tensor/cpu_dtype.go:438-446 ->
  * tensor/cpu_quant_q8.go:125-259): x rows are quantized on the device to Q8 blocks of the
- * weight's block size (quantizeQ8), integer block sums are exact int32 (int8 MFMA for M >= 8: q4_k, q6_k, and
- * q4_0 when the row's block count is a multiple of 8; packed int8 dot products otherwise), and the per-block
+ * weight's block size (quantizeQ8), integer block sums are exact int32 (int8 MFMA: q4_k and q6_k at every M, q4_0
+ * from M = 8 when the row's block count is a multiple of 8; packed int8 dot products otherwise), and the per-block
  * fp32 epilogue follows the reference order, so outputs are bit-identical to the CPU path.
  * Rows holding NaN/Inf use the fp32 path for that row only. dtype must be q4, q4_k or q6_k
  * (QuantActSupported, tensor/cpu_quant_q8.go:122), else TRHIP_ERR_UNSUPPORTED. */
@@ -174,7 +174,7 @@ int trhip_gemm_q_actq(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64
  * the same operator). TRHIP_MODE_EXACT is trhip_gemm_q_actq. TRHIP_MODE_FAST keeps the quantized activations and
  * the exact int32 block sums (isum, msum) and fuses the per-block fp32 epilogue (two fma instead of two products,
  * a difference and a sum) on the q4_k matrix-core kernels: deterministic and within 1e-4 of the exact result,
- * |a - b| / (1 + |b|); other dtypes and small M run exact. */
+ * |a - b| / (1 + |b|); other dtypes run exact. */
 int trhip_gemm_q_actq_mode(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x,
                            float *c, int64_t M, int64_t K, int accumulate, int mode);
 

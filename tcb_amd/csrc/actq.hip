@@ -37,12 +37,8 @@ __global__ __launch_bounds__(256) void quantize_q8_kernel(const float *__restric
     const int64_t blk_id = gtc / TPB;  // = m * nbk + b
     const int64_t off = blk_id * BLK + 4 * l4;  // element offset in x (rows are contiguous: m*K + b*BLK)
     float4 v = *reinterpret_cast<const float4 *>(x + off);
-    float a = 0.0f;
-    float av[4] = {fabsf(v.x), fabsf(v.y), fabsf(v.z), fabsf(v.w)};
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-        if (av[i] > a) a = av[i];
-    int bad = ((v.x - v.x) != 0.0f) | ((v.y - v.y) != 0.0f) | ((v.z - v.z) != 0.0f) | ((v.w - v.w) != 0.0f);
+    float a = amax4(v);
+    int bad = non_finite4(v);
 #pragma unroll
     for (int s = 1; s < TPB; s <<= 1) {
         float o = __shfl_xor(a, s);
@@ -51,24 +47,9 @@ __global__ __launch_bounds__(256) void quantize_q8_kernel(const float *__restric
     }
     if (!live) return;
     if (l4 == 0) bad_blk[blk_id] = (uint8_t)(bad != 0);
-    float id = 127.0f / a;
     float dv;
-    int c[4];
-    if (!(a > 0.0f) || (id - id) != 0.0f) {
-        dv = 0.0f;
-        c[0] = c[1] = c[2] = c[3] = 0;
-    } else {
-        dv = a / 127.0f;
-        float xv[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            float t = rintf(xv[i] * id);
-            t = fminf(fmaxf(t, -127.0f), 127.0f);
-            c[i] = (int)t;
-        }
-    }
-    uint32_t packed = (uint32_t)(c[0] & 0xFF) | ((uint32_t)(c[1] & 0xFF) << 8) | ((uint32_t)(c[2] & 0xFF) << 16) |
-                      ((uint32_t)(c[3] & 0xFF) << 24);
+    int s16;
+    const uint32_t packed = q8_codes(v, a, dv, s16);
     const int64_t m = blk_id / nbk, b = blk_id % nbk;
     if (TILED) {
         *reinterpret_cast<uint32_t *>(q + tiled_q(m, b, nbk, 4 * l4)) = packed;
@@ -77,7 +58,6 @@ __global__ __launch_bounds__(256) void quantize_q8_kernel(const float *__restric
         *reinterpret_cast<uint32_t *>(q + off) = packed;
         if (l4 == 0) d[blk_id] = dv;
     }
-    int s16 = c[0] + c[1] + c[2] + c[3];
     s16 += __shfl_xor(s16, 1);
     s16 += __shfl_xor(s16, 2);
     if (!TILED && (l4 & 3) == 0) bs[off / 16] = (int16_t)s16;
@@ -104,8 +84,8 @@ __device__ __forceinline__ int sdot4(uint32_t a, uint32_t b, int c) {
     return __builtin_amdgcn_sdot4((int)a, (int)b, c, false);
 }
 
-// One thread per output (m, n); blocks in order. Correct for every M; the int8-MFMA kernel
-// (actq_mfma.hip) takes the large-M shapes.
+// One thread per output (m, n); blocks in order. Correct for every M: what the matrix-core kernels do not take (q4_0 of
+// few rows or a block count that is no multiple of 8; q4_k and q6_k whose padded tiles do not fit the static scratch).
 template <int DT, bool ACC>
 __global__ __launch_bounds__(256) void actq_valu_kernel(const Planes p, int64_t N, int64_t row0, int64_t K,
                                                         const float *__restrict__ x, const int8_t *__restrict__ q,
@@ -246,7 +226,8 @@ int launch_quantize_q8(trhip_ctx *ctx, const float *x, int64_t M, int64_t K, int
     return launch_check(ctx, "quantize_q8");
 }
 
-// Below this many activation rows the thread-per-output kernel wins (the MFMA tile is 128 rows).
+// q4_k reaches this below actqw.hip's share only with a forced launch shape, or where its padded tiles do not fit the
+// static scratch.
 constexpr int64_t kActqMfmaMinRows = 8;
 
 int launch_actq_mfma(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c,
@@ -266,7 +247,6 @@ int launch_actq(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, 
         if (M >= kActqMfmaMinRows && sj) return launch_actq_mfma(ctx, w, row0, N, x, c, M, acc, q, d, sj, bad, fast);
         return run_valu<kQ4K>(ctx, w, row0, N, x, c, M, acc, q, d, bs, bad);
     case kQ6K:
-        if (actq6_mfma_applies(M, N, row0, w->K)) return launch_actq6_mfma(ctx, w, row0, N, x, c, M, acc, q, d, bad);
         return run_valu<kQ6K>(ctx, w, row0, N, x, c, M, acc, q, d, bs, bad);
     }
     return fail(ctx, TRHIP_ERR_UNSUPPORTED, "actq: dtype must be q4, q4_k or q6_k");

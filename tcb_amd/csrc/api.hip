@@ -1021,23 +1021,35 @@ int trhip_quantize_q8(trhip_ctx *ctx, const float *x, int64_t M, int64_t K, int 
 
 namespace {
 
+// How an act-quant call runs: on row-major quantized activations (launch_actq), or on the tiled ones (q4_k, q6_k) with
+// prefill.hip's 128 x 256 tiles or with actqw.hip's blocks dealt over waves.
+enum class ActqRoute { rows, blocks, tiles };
+
+ActqRoute actq_route(const trhip_ctx *ctx, int dtype, int64_t M, int64_t N, int64_t row0, int64_t K) {
+    if (prefill_tiles_apply(dtype, M, N, row0, K)) return ActqRoute::tiles;
+    const bool forced = ctx->force_actq_tm || ctx->force_actq_slices;  // the 64-row q4_k kernel's launch shape
+    return actq_blocks_applies(dtype, M, N) && !(dtype == TRHIP_Q4K && forced) ? ActqRoute::blocks : ActqRoute::rows;
+}
+
 // Scratch layout of the act-quant operator: q [M][K] int8, d [M][K/blk] fp32, bs [M][K/16] int16, one NaN/Inf flag
 // byte per activation block, for q4_k the f16 msum operands [M][K/256][16], and an aligned copy of x when x is not
-// 16-byte aligned. When a prefill kernel (q4_k, q6_k) takes the shape (tiles), q, d and the q4_k msum operands are in
-// its tiled layout over rows padded to a multiple of 128, and there are no 16-sums.
+// 16-byte aligned. On the tiled routes q, d and the q4_k msum operands are in the tiled layout over rows padded to whole
+// tiles (32 rows) or prefill tiles (128), and there are no 16-sums.
 struct ActqLayout {
     size_t o_q = 0, o_d = 0, o_bs = 0, o_fl = 0, o_sj = 0, o_x = 0, total = 0;
-    bool copy_x = false, tiles = false;
+    bool copy_x = false;
+    ActqRoute route = ActqRoute::rows;
 };
 
-ActqLayout actq_layout(int dtype, int64_t M, int64_t N, int64_t row0, int64_t K, const float *x) {
+ActqLayout actq_layout(ActqRoute route, int dtype, int64_t M, int64_t K, const float *x) {
     ActqLayout l;
+    l.route = route;
     const int64_t nb = K / block_elems(dtype);
-    l.tiles = prefill_tiles_apply(dtype, M, N, row0, K);
-    const int64_t Mq = l.tiles ? (M + kPrefillRowPad - 1) / kPrefillRowPad * kPrefillRowPad : M;
+    const bool tiled = route != ActqRoute::rows;
+    const int64_t pad = route == ActqRoute::tiles ? kPrefillRowPad : tiled ? 32 : 1, Mq = (M + pad - 1) / pad * pad;
     l.o_d = align_up(l.o_q + (size_t)(Mq * K), 256);
     l.o_bs = align_up(l.o_d + (size_t)(Mq * nb) * sizeof(float), 256);
-    l.o_fl = align_up(l.o_bs + (l.tiles ? 0 : (size_t)(M * (K / 16)) * sizeof(int16_t)), 256);
+    l.o_fl = align_up(l.o_bs + (tiled ? 0 : (size_t)(M * (K / 16)) * sizeof(int16_t)), 256);
     l.o_sj = align_up(l.o_fl + (size_t)(M * nb), 256);
     l.o_x = align_up(l.o_sj + (dtype == TRHIP_Q4K ? (size_t)(Mq * nb) * 32 : 0), 256);
     l.copy_x = reinterpret_cast<uintptr_t>(x) % 16 != 0;
@@ -1074,9 +1086,12 @@ int actq_run(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, con
         if (e != hipSuccess) return hip_fail(ctx, e, "gemm_q_actq: align x");
         xa = tmp;
     }
-    if (l.tiles) {
-        int st = launch_quantize_tiles(ctx, xa, M, K, q, d, sj, bad);
+    if (l.route != ActqRoute::rows) {
+        int st = TRHIP_OK;
+        if (l.route == ActqRoute::tiles || !actq_blocks_quantizes(M)) st = launch_quantize_tiles(ctx, xa, M, K, q, d, sj, bad);
         if (st != TRHIP_OK) return st;
+        if (l.route == ActqRoute::blocks)
+            return launch_actq_blocks(ctx, w, row0, N, xa, c, M, accumulate != 0, q, d, sj, bad, fast);
         if (w->dtype == TRHIP_Q6K) return launch_prefill_q6k(ctx, w, row0, N, xa, c, M, accumulate != 0, q, d, bad);
         return launch_prefill_q4k(ctx, w, row0, N, xa, c, M, accumulate != 0, q, d, sj, bad, fast);
     }
@@ -1122,7 +1137,7 @@ int trhip_gemm_q_actq_mode(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, 
     if (r) return st;
     DevGuard g(ctx);
     if (K == 0) return accumulate ? TRHIP_OK : zero_f32(ctx, c, M * N);
-    const ActqLayout l = actq_layout(w->dtype, M, N, row0, K, x);
+    const ActqLayout l = actq_layout(actq_route(ctx, w->dtype, M, N, row0, K), w->dtype, M, K, x);
     uint8_t *ws = static_cast<uint8_t *>(workspace(ctx, l.total, &st));
     if (!ws) return st;
     return actq_run(ctx, w, row0, N, x, c, M, K, accumulate, ws, l, mode == TRHIP_MODE_FAST);
@@ -1140,7 +1155,10 @@ int trhip_gemm_q_actq_noalloc(trhip_ctx *ctx, const trhip_wstore *w, int64_t row
     const int r = actq_check(ctx, w, row0, N, x, c, M, K, "gemm_q_actq_noalloc", &st);
     if (r) return st;
     if (K != 0) {
-        const ActqLayout l = actq_layout(w->dtype, M, N, row0, K, x);
+        ActqLayout l = actq_layout(actq_route(ctx, w->dtype, M, N, row0, K), w->dtype, M, K, x);
+        // tiles padded past the scratch: the row-major layout, which pads nothing, may still fit
+        if (l.total > (size_t)TRHIP_NOALLOC_SCRATCH_BYTES && l.route == ActqRoute::blocks)
+            l = actq_layout(ActqRoute::rows, w->dtype, M, K, x);
         if (l.total > (size_t)TRHIP_NOALLOC_SCRATCH_BYTES)
             return fail(ctx, TRHIP_ERR_INVALID,
                         "gemm_q_actq_noalloc: M x K needs " + std::to_string(l.total) + " bytes of scratch; the static "

@@ -70,20 +70,6 @@ __device__ __forceinline__ float pf_epilogue(float acc, int p0, int p1, float cm
     return acc + tt * d8;
 }
 
-// Eight integers below 64 (the bytes of lo, then hi) times c (1 or 64) as f16: v_perm_b32 places each byte under
-// 0x64, giving the f16 value 1024 + v; subtracting 1024 and multiplying by c are both exact (v c <= 4032). (A fused
-// (1024 + v) c - 1024 c is not usable: -1024 * 64 is beyond the f16 range.)
-__device__ __forceinline__ v8h small_f16x8(uint32_t lo, uint32_t hi, _Float16 c) {
-    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    const h2 cc = (h2){c, c}, off = (h2){(_Float16)(-1024.0f), (_Float16)(-1024.0f)};
-    auto pair = [&](uint32_t v, uint32_t sel) {
-        const h2 x = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, v, sel));
-        return __builtin_bit_cast(uint32_t, (x + off) * cc);
-    };
-    return __builtin_bit_cast(v8h, make_uint4(pair(lo, 0x04010400u), pair(lo, 0x04030402u), pair(hi, 0x04010400u),
-                                              pair(hi, 0x04030402u)));
-}
-
 // One 32-row tile of a block: 16 int8 MFMAs into (c0, c1), and between them the epilogue of the pending tile held in
 // (p0, p1) with msum pcm, the pending block's d, dmin and the d8 of its rows (pd8, this lane's rows at + 8 (v / 4)
 // + (v % 4)). The pending sums are final only once the previous tile's last MFMAs have completed, so the first MFMA
@@ -347,31 +333,6 @@ struct Pf6 {
     static constexpr size_t LDS = DOFF + 3 * D + (TM + 1) * sizeof(int);
 };
 static_assert(Pf6::LDS <= 160 * 1024, "one workgroup per CU");
-
-typedef short pf_s2 __attribute__((ext_vector_type(2)));
-
-// Chunk kc's two B operands for lane (r, h): elements 32 kc + 16 h .. + 15 of the row, the four 4-element groups
-// e = 2 tt + hh (tt, hh in 0..1) from ql dword L[e] (nibble half k / 2) and qh dword H[e] (bit pair k = kc % 4), all
-// in sub-block 2 kc + h with signed scale sc. Per group: the codes c as bytes, spread to 16-bit pairs, v = c sc - 32 sc
-// by packed 16-bit multiply-adds, then the bytes of v >> 7 (h) and of v & 127 (l).
-__device__ __forceinline__ void q6_planes(const uint32_t (&L)[4], const uint32_t (&H)[4], int k, int sc, v4i &lo,
-                                          v4i &hi) {
-    const pf_s2 S = (pf_s2){(short)sc, (short)sc}, O = (pf_s2){(short)(-32 * sc), (short)(-32 * sc)};
-    uint32_t lb[4], hb[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const uint32_t lw = (k >> 1) ? (L[e] >> 4) : L[e];
-        const uint32_t hw = k == 0 ? (H[e] << 4) : k == 1 ? (H[e] << 2) : k == 2 ? H[e] : (H[e] >> 2);
-        const uint32_t C = (lw & 0x0F0F0F0Fu) | (hw & 0x30303030u);  // codes 0..63
-        const pf_s2 c01 = __builtin_bit_cast(pf_s2, __builtin_amdgcn_perm(0u, C, 0x0c010c00u));
-        const pf_s2 c23 = __builtin_bit_cast(pf_s2, __builtin_amdgcn_perm(0u, C, 0x0c030c02u));
-        const uint32_t v01 = __builtin_bit_cast(uint32_t, c01 * S + O), v23 = __builtin_bit_cast(uint32_t, c23 * S + O);
-        lb[e] = __builtin_amdgcn_perm(v23, v01, 0x06040200u) & 0x7F7F7F7Fu;  // low bytes, low 7 bits: v & 127
-        hb[e] = __builtin_amdgcn_perm(v23 >> 7, v01 >> 7, 0x06040200u);     // bits 7..14 of each v: v >> 7
-    }
-    lo = (v4i){(int)lb[0], (int)lb[1], (int)lb[2], (int)lb[3]};
-    hi = (v4i){(int)hb[0], (int)hb[1], (int)hb[2], (int)hb[3]};
-}
 
 template <bool ACC, bool PROBE = false>  // PROBE: as for prefill_q4k
 __global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_q6k(

@@ -272,6 +272,36 @@ __device__ __forceinline__ float exact_dot_row(const Planes p, int64_t row, cons
     return exact_dot_range<DT>(p, row, xr, 0, K);
 }
 
+// quantizeQ8 (tensor/cpu_quant_q8.go:39-68) for four elements v of an activation block whose largest |x| is a (a NaN
+// never enters it): the codes as bytes, the block's scale and the codes' sum. id = fl(127 / a); a zero block or an
+// infinite id gives zero codes and scale, else d = fl(a / 127) and code = clamp(rne(fl(x id)), +-127). Division is IEEE
+// (correctly rounded), rintf is round-to-nearest-even, nothing is fused.
+__device__ __forceinline__ float amax4(const float4 &v) {
+    float a = 0.0f;
+    const float av[4] = {fabsf(v.x), fabsf(v.y), fabsf(v.z), fabsf(v.w)};
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        if (av[i] > a) a = av[i];
+    return a;
+}
+__device__ __forceinline__ int non_finite4(const float4 &v) {
+    return ((v.x - v.x) != 0.0f) | ((v.y - v.y) != 0.0f) | ((v.z - v.z) != 0.0f) | ((v.w - v.w) != 0.0f);
+}
+__device__ __forceinline__ uint32_t q8_codes(const float4 &v, float a, float &d, int &sum) {
+    const float id = 127.0f / a;
+    const float xv[4] = {v.x, v.y, v.z, v.w};
+    int c[4] = {0, 0, 0, 0};
+    d = 0.0f;
+    if (a > 0.0f && (id - id) == 0.0f) {
+        d = a / 127.0f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) c[i] = (int)fminf(fmaxf(rintf(xv[i] * id), -127.0f), 127.0f);
+    }
+    sum = c[0] + c[1] + c[2] + c[3];
+    return (uint32_t)(c[0] & 0xFF) | ((uint32_t)(c[1] & 0xFF) << 8) | ((uint32_t)(c[2] & 0xFF) << 16) |
+           ((uint32_t)(c[3] & 0xFF) << 24);
+}
+
 // Tiled activation layout of the q4_k prefill kernel (prefill.hip), per 32-row tile mt = m / 32 and block b, in
 // the operand order of its MFMAs so that each 1 KB piece is one coalesced load straight into LDS:
 //   codes   : 8 KB = chunk kc (32 elements of sub-block kc) x lane (r + 32 h) x 16 bytes (elements 32 kc + 16 h + i)
@@ -401,6 +431,14 @@ int launch_prefill_q4k(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int6
 // q6_k weights on the same tiles (prefill.hip), always exact.
 int launch_prefill_q6k(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c,
                        int64_t M, bool acc, const int8_t *qt, const float *dt, const uint8_t *bad);
+// q4_k and q6_k weights over the same tiled activations (rows padded to 32), blocks dealt over waves (actqw.hip): whether
+// it takes the shape, whether it quantizes x itself (the tiled buffers are then not read), the kernels; fast as for
+// launch_prefill_q4k.
+bool actq_blocks_applies(int dtype, int64_t M, int64_t N);
+bool actq_blocks_quantizes(int64_t M);
+int launch_actq_blocks(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c,
+                       int64_t M, bool acc, const int8_t *qt, const float *dt, const uint16_t *st, const uint8_t *bad,
+                       bool fast);
 // 16-bit activations / outputs (io16.hip): dst[i] = widen(src[i]) and dst[i] = round(src[i]) for n elements.
 int launch_widen16(trhip_ctx *ctx, const uint16_t *src, float *dst, int64_t n, int io);
 int launch_round16(trhip_ctx *ctx, const float *src, uint16_t *dst, int64_t n, int io);
@@ -421,12 +459,9 @@ int launch_mfma_probe(trhip_ctx *ctx, int valu_per_mfma, int waves_per_simd, int
 // io: TRHIP_F32, or f16 / bf16 x and c (read and written directly; not with swi).
 int launch_rows16(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const void *x, void *c,
                       int64_t M, bool acc, float *swi = nullptr, int io = TRHIP_F32);
-// q4_0 and q6_k act-quant on int8 matrix cores (actq4.hip, actq6.hip): whether each takes the shape, and the kernel.
+// q4_0 act-quant on int8 matrix cores (actq4.hip): whether it takes the shape, and the kernel.
 bool actq4_mfma_applies(int64_t M, int64_t N, int64_t row0, int64_t K);
 int launch_actq4_mfma(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c,
-                      int64_t M, bool acc, const int8_t *q, const float *d, const uint8_t *bad);
-bool actq6_mfma_applies(int64_t M, int64_t N, int64_t row0, int64_t K);
-int launch_actq6_mfma(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c,
                       int64_t M, bool acc, const int8_t *q, const float *d, const uint8_t *bad);
 int launch_actq(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c,
                 int64_t M, bool acc, const int8_t *q, const float *d, const int16_t *bs, const uint8_t *bad,
