@@ -14,7 +14,7 @@ OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libtrhip.so")
 
 SOURCES = ["api.hip", "wstore.hip", "gemv.hip", "gemv_fast.hip", "gemm_rows.hip", "actq.hip", "actq_mfma.hip",
-           "swiglu.hip", "probe.hip", "prefill.hip", "actqw.hip", "rows16.hip", "actq4.hip",
+           "swiglu.hip", "probe.hip", "prefill.hip", "actqw.hip", "rows16.hip", "actq4.hip", "fastg.hip",
            "io16.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

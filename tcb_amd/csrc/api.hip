@@ -898,11 +898,14 @@ int trhip_gemm_q(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N,
     }
     // fast mode (tolerance) on matrix cores: q4_k from M = 5 (up to 4 rows the exact kernel's 4-row tiles are as
     // fast), up to 16 rows in one launch over f16 activation pairs, more over fixed-point digits; q4_0 up to 16 rows
-    // over f16 activation pairs; q6_k from M = 2; q8_0 and q4_0 beyond 16 rows run exact
+    // over f16 activation pairs; q6_k from M = 2; every dtype at many rows on f16 matrix cores (fast_gemm_applies); other
+    // calls run exact
     if (mode == TRHIP_MODE_FAST && M <= 16 && ((w->dtype == TRHIP_Q4K && M > 4) || (w->dtype == TRHIP_Q4 && M > 1))) {
         const int r = launch_rows16(ctx, w, row0, N, x, c, M, accumulate != 0);
         if (r != -1) return r;
     }
+    if (mode == TRHIP_MODE_FAST && fast_gemm_applies(w->dtype, M, N, K))
+        return launch_fast_gemm(ctx, w, row0, N, x, c, M, accumulate != 0);
     if (mode == TRHIP_MODE_FAST && ((w->dtype == TRHIP_Q4K && M > 4) || (w->dtype == TRHIP_Q6K && M > 1)))
         return launch_gemm_rows_fast(ctx, w, row0, N, x, c, M, accumulate != 0);
     return launch_gemm_rows(ctx, w, row0, N, x, c, M, accumulate != 0);
@@ -999,6 +1002,8 @@ int trhip_gemm_q_swiglu(trhip_ctx *ctx, const trhip_wstore *w, const float *x, f
         const int r = launch_rows16(ctx, w, 0, w->N, x, nullptr, M, false, out);
         if (r != -1) return r;
     }
+    if (mode == TRHIP_MODE_FAST && K > 0 && fast_gemm_applies(w->dtype, M, w->N, K))
+        return launch_fast_gemm(ctx, w, 0, w->N, x, gu, M, false, out);
     if (mode == TRHIP_MODE_FAST && K > 0 && ((w->dtype == TRHIP_Q4K && M > 4) || (w->dtype == TRHIP_Q6K && M > 1)))
         return launch_gemm_rows_fast(ctx, w, 0, w->N, x, gu, M, false, out);
     if ((st = trhip_gemm_q(ctx, w, 0, w->N, x, gu, M, K, 0, mode)) != TRHIP_OK) return st;

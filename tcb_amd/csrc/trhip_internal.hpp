@@ -417,6 +417,11 @@ int launch_gemm_rows(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_
 // into the slice sum when K is split (c is then not written), else after it
 int launch_gemm_rows_fast(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c,
                           int64_t M, bool acc, float *swi = nullptr);
+// Fast mode for many rows, every dtype, on f16 matrix cores (fastg.hip): whether it takes the shape; swi as for
+// launch_gemm_rows_fast.
+bool fast_gemm_applies(int dtype, int64_t M, int64_t N, int64_t K);
+int launch_fast_gemm(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c, int64_t M,
+                     bool acc, float *swi = nullptr);
 int launch_quantize_q8(trhip_ctx *ctx, const float *x, int64_t M, int64_t K, int blk, int8_t *q, float *d,
                        int16_t *bs, uint8_t *bad, uint16_t *sj);
 int launch_read_probe(trhip_ctx *ctx, const void *p, int64_t bytes);

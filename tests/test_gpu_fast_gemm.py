@@ -1,0 +1,114 @@
+"""Fast mode at many rows (fastg.hip, every dtype): two f16 terms of x on the matrix cores.
+
+Bounds. Against float64, the product of the dequantized weights: x is split to 2^-23 of each element, products are
+exact, and what rounds is fp32 sums no longer than the exact mode's chains, so the relative error (2-norm) stays below
+the exact mode's own on the same inputs (measured 0.3 to 0.7 of it); the test allows equality. Per element the header's
+bound, |a - b| / (1 + |b|) <= 1e-5 (q8_0, q4_0) / 1e-4 (q4_k, q6_k) of the oracle, at x1 and x1000."""
+import numpy as np
+import pytest
+
+import oracle as O
+from conftest import rel_err, same_bits
+from tcb_amd import MODE_FAST, Q4, Q4K, Q6K, Q8, synth
+
+pytestmark = pytest.mark.gpu
+
+TOL = {Q8: 1e-5, Q4: 1e-5, Q4K: 1e-4, Q6K: 1e-4}
+
+
+def _call(backend, w, x, off, N, K, c0, row0, acc):
+    M = x.shape[0]
+    xb = backend.ctx.alloc(x.nbytes + 64)
+    xb.upload(x, byte_offset=off)
+    cb = backend.ctx.to_device(c0)
+    (backend.Gemm if acc else backend.GemmSet)(M, N, K, (xb, off), w, cb, row0=row0, mode=MODE_FAST)
+    got = cb.download(np.float32, M * N).reshape(M, N)
+    xb.free()
+    cb.free()
+    return got
+
+
+# q8_0 / q4_0: 32-, 64- and 128-row tiles, ragged rows and columns, ragged 64-element steps, K slices; K below 256 (exact)
+SMALL = [(49, 33, 32, 0), (64, 257, 96, 3), (65, 256, 288, 0), (128, 300, 992, 1), (129, 255, 4096, 0), (50, 1030, 544, 2),
+         (17, 14500, 4096, 0), (33, 8000, 4096, 0)]
+# k-quants: the smallest products that take this path
+LARGE = {Q4K: [(129, 14336, 4096, 0), (460, 2051, 8192, 1), (64, 29000, 4096, 0), (2100, 14000, 256, 0)],
+         Q6K: [(130, 8000, 4096, 0), (260, 2051, 7680, 1), (32, 31000, 4096, 0), (1200, 13100, 256, 0)]}
+
+
+@pytest.mark.parametrize("dt,M,N,K,row0", [(dt, *s) for dt in (Q8, Q4) for s in SMALL] +
+                         [(dt, *s) for dt in (Q4K, Q6K) for s in LARGE[dt]])
+def test_fast_gemm(backend, dt, M, N, K, row0):
+    raw = synth.quant_weights(dt, row0 + N, K, seed=M + K, outliers=0.01)
+    w = backend.FromQuantized(dt, raw, row0 + N, K)
+    rows = np.ascontiguousarray(raw.reshape(row0 + N, -1)[row0:]).reshape(-1)
+    x = synth.activations(M, K, seed=N)
+    x[M // 2] = 0
+    x[1] *= np.float32(1000)
+    x[M - 1, K - 1] = np.nan
+    c0 = synth.activations(M, N, seed=3)
+    pick = sorted({0, 1, M // 2, M - 2, M - 1, min(M - 1, 31), min(M - 1, 32), min(M - 1, 63), min(M - 1, 64)})
+    deq = O.dequant(dt, rows).reshape(N, K)
+    for acc, off in ((False, 0), (True, 4)):
+        got = _call(backend, w, x, off, N, K, c0, row0, acc)
+        same_bits(got, _call(backend, w, x, off, N, K, c0, row0, acc))
+        want = O.quant_gemm(dt, len(pick), N, K, x[pick], rows, c0[pick].reshape(-1) if acc else None).reshape(len(pick), N)
+        for i, m in enumerate(pick):
+            if m == M - 1:
+                assert np.isnan(got[m]).all() and np.isnan(want[i]).all()
+                continue
+            scale = np.float32(1000 if m == 1 else 1)
+            assert rel_err(got[m] / scale, want[i] / scale) <= TOL[dt], (m, acc)
+            if m == M // 2:
+                same_bits(got[m], c0[m] if acc else np.zeros(N, np.float32))
+        if not acc:
+            fin = [i for i, m in enumerate(pick) if m != M - 1]
+            truth = x[pick][fin].astype(np.float64) @ deq.astype(np.float64).T
+            err = [np.linalg.norm(y - truth) / np.linalg.norm(truth) for y in (got[pick][fin], want[fin])]
+            assert err[0] <= err[1], err
+    w.release()
+
+
+@pytest.mark.parametrize("dt", [Q8, Q4, Q4K, Q6K])
+def test_fast_gemm_ranges(backend, dt):
+    """One exponent per row: rows of huge, tiny and subnormal values, one huge element among tiny ones, Inf rows."""
+    M, N, K = 300, (1024 if dt in (Q8, Q4) else 6600), 4096
+    raw = synth.quant_weights(dt, N, K, seed=8, outliers=0.01)
+    w = backend.FromQuantized(dt, raw, N, K)
+    rng = np.random.default_rng(3)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x[0] *= 1e30
+    x[1] *= np.float32(1e-30)
+    x[2] = x[2] * np.float32(1e-40)
+    x[3, 5] = 1e4
+    x[4, :256] *= np.float32(1e-20)
+    x[5, 9] = np.inf
+    x[6, 0] = -np.inf
+    got = _call(backend, w, x, 0, N, K, np.zeros((M, N), np.float32), 0, False)
+    want = O.quant_gemm(dt, 7, N, K, x[:7], raw).reshape(7, N)
+    for m in range(7):
+        assert np.array_equal(np.isnan(got[m]), np.isnan(want[m]))
+        if m >= 5:
+            assert np.array_equal(got[m][~np.isnan(want[m])], want[m][~np.isnan(want[m])])
+            continue
+        amax = float(np.max(np.abs(x[m])))
+        if m == 2:  # results in the subnormal range: units of the last place
+            assert float(np.max(np.abs(got[m].astype(np.float64) - want[m]))) <= K * 2.0 ** -149
+        else:
+            assert rel_err(got[m] / np.float32(amax), want[m] / np.float32(amax)) <= TOL[dt], m
+    w.release()
+
+
+@pytest.mark.parametrize("dt,M,I,K", [(Q8, 70, 300, 992), (Q4, 300, 130, 4096), (Q4K, 512, 1800, 4608), (Q6K, 300, 2000, 4096)])
+def test_fast_gemm_swiglu(backend, dt, M, I, K):
+    """The gate applied in the slice sum or after the kernel gives the bits of the product followed by the gate."""
+    raw = synth.quant_weights(dt, 2 * I, K, seed=I, outliers=0.01)
+    w = backend.FromQuantized(dt, raw, 2 * I, K)
+    x = synth.activations(M, K, seed=K)
+    gu = _call(backend, w, x, 0, 2 * I, K, np.zeros((M, 2 * I), np.float32), 0, False)
+    xb, ob = backend.ctx.to_device(x), backend.ctx.alloc(M * I * 4)
+    backend.GemmSwiGLU(M, K, xb, w, ob, mode=MODE_FAST)
+    same_bits(ob.download(np.float32, M * I), O.swiglu(gu, M, I).reshape(-1))
+    for b in (xb, ob):
+        b.free()
+    w.release()
