@@ -329,7 +329,9 @@ struct Tiles {
 // The same chains on the matrix cores, a pass of Tiles<MT>::kRows activation rows at a time, in ascending k from +0
 // as the CPU kernel does. Activation rows past M repeat row M - 1; their results are dropped.
 //
-// Workgroup (blockIdx.x, blockIdx.y) covers rows 64 blockIdx.x .. +63 and chunks [cps blockIdx.y, + cps). A wave
+// Workgroup (blockIdx.x, blockIdx.y, blockIdx.z) covers rows 64 blockIdx.x .. +63, chunks [cps blockIdx.y, + cps) and
+// every gridDim.z-th pass from blockIdx.z. MT = -1: passes of 32 rows, two 16-row tiles on one decoding of the weights
+// (the tiles share the LDS tile of activations in turn, so the LDS is that of one). A wave
 // stages its chunk's weight images in LDS (loaded during its previous chunk) and each 32-wide group of activations
 // (loaded a few groups ahead) in a 16 x 32 LDS tile that its lanes read back as A operands. With partial == null
 // the workgroup covers every chunk and adds the chain results to `part` in chunk order in LDS; otherwise each
@@ -339,8 +341,11 @@ __global__ __launch_bounds__(64 * W) void gemm_rows_mfma(const Planes p, const f
                                                          float *__restrict__ c, float *__restrict__ partial, int64_t N,
                                                          int64_t row0, int64_t M, int64_t K, int64_t cps) {
     using I = Image<DT>;
-    constexpr int XD = DT == kQ8 ? 1 : DT == kQ6K ? 2 : 4;  // activation groups in flight (larger images leave fewer registers)
-    static_assert(16 * kRPitch * 4 <= 64 * I::kPitch, "chain results reuse the wave's image space");
+    using TL = Tiles<MT < 0 ? 0 : MT>;
+    constexpr int NT = MT < 0 ? 2 : 1, MP = NT * TL::kRows;  // tiles and activation rows of a pass
+    // activation groups in flight (larger images and two tiles leave fewer registers)
+    constexpr int XD = DT == kQ8 ? 1 : DT == kQ6K || NT == 2 ? 2 : 4;
+    static_assert(NT * 16 * kRPitch * 4 <= 64 * I::kPitch, "chain results reuse the wave's image space");
     __shared__ __align__(16) uint8_t wsl[W][64 * I::kPitch];
     __shared__ __align__(16) float xsl[W][16 * kXPitch];
     const int lane = threadIdx.x & 63;
@@ -353,17 +358,22 @@ __global__ __launch_bounds__(64 * W) void gemm_rows_mfma(const Planes p, const f
     uint8_t *ws = wsl[cw];
     float *xs = xsl[cw];
     const uint8_t *img = ws + lane * I::kPitch;
-    constexpr int MP = Tiles<MT>::kRows;
-    for (int64_t m0 = 0; m0 < M; m0 += MP) {
+    for (int64_t m0 = (int64_t)blockIdx.z * MP; m0 < M; m0 += (int64_t)gridDim.z * MP) {
         const int64_t mb = (M - m0) < MP ? (M - m0) : MP;
-        const float *xp[2];  // x piece P = 64 i + lane: activation row P / 8, floats 4 (P % 8) .. +3 of a group
+        const bool two = NT == 2 && mb > 16;  // the pass has rows for its second tile
+        const float *xp[2 * NT];  // x piece P = 64 i + lane: activation row P / 8, floats 4 (P % 8) .. +3 of a group
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
+        for (int i = 0; i < 2 * NT; i++) {
             const int P = 64 * i + lane, m = P >> 3;
             xp[i] = x + (m0 + (m < mb ? m : mb - 1)) * K + 4 * (P & 7);
         }
-        f32x4 xg[XD][2];  // activations of the next XD groups; group g of every chunk uses slot g % XD
-        constexpr int PR = 16 / W;
+        f32x4 xg[XD][2 * NT];  // activations of the next XD groups; group g of every chunk uses slot g % XD
+        auto fetch = [&](f32x4(&v)[2 * NT], int64_t k) {
+#pragma unroll
+            for (int i = 0; i < 2 * NT; i++)
+                if (i < 2 || two) v[i] = *reinterpret_cast<const f32x4 *>(xp[i] + k);
+        };
+        constexpr int PR = 16 * NT / W;
         float part[PR];
 #pragma unroll
         for (int j = 0; j < PR; j++) part[j] = 0.0f;
@@ -374,10 +384,7 @@ __global__ __launch_bounds__(64 * W) void gemm_rows_mfma(const Planes p, const f
             const int ng0 = (int)(((K - k0) < 256 ? (K - k0) : 256) / 32);
 #pragma unroll
             for (int g = 0; g < XD; g++)
-                if (g < ng0) {
-#pragma unroll
-                    for (int i = 0; i < 2; i++) xg[g][i] = *reinterpret_cast<const f32x4 *>(xp[i] + k0 + 32 * g);
-                }
+                if (g < ng0) fetch(xg[g], k0 + 32 * g);
         }
         for (int64_t c0 = cb; c0 < ce; c0 += W) {
             const int64_t pc = c0 + cw;
@@ -389,40 +396,55 @@ __global__ __launch_bounds__(64 * W) void gemm_rows_mfma(const Planes p, const f
                 const bool more = pc + W < ce;
                 const int64_t kx = (pc + W) * 256;  // the wave's next chunk
                 const int ngx = more ? (int)(((K - kx) < 256 ? (K - kx) : 256) / 32) : 0;
-                Tiles<MT> tl;
-                tl.zero();
+                TL tl[NT];
+#pragma unroll
+                for (int h = 0; h < NT; h++) tl[h].zero();
                 static_for<0, 8>([&](auto G) {
                     constexpr int gi = decltype(G)::value;
                     constexpr int sl = gi % XD;
                     if (gi < ngroups) {
-                        __builtin_amdgcn_wave_barrier();
+                        auto put_x = [&](int h) {  // tile h's activations of this group
+                            __builtin_amdgcn_wave_barrier();
 #pragma unroll
-                        for (int i = 0; i < 2; i++) {
-                            const int P = 64 * i + lane;
-                            *reinterpret_cast<f32x4 *>(xs + (P >> 3) * kXPitch + 4 * (P & 7)) = xg[sl][i];
-                        }
+                            for (int i = 0; i < 2; i++) {
+                                const int P = 64 * i + lane;
+                                *reinterpret_cast<f32x4 *>(xs + (P >> 3) * kXPitch + 4 * (P & 7)) = xg[sl][2 * h + i];
+                            }
+                        };
                         // the activations XD groups on, then (once a chunk) the next chunk's weights, are in flight
                         // during the arithmetic of the groups before them
-                        constexpr int gn = gi + XD;
-                        if (gn < ngroups || gn - ngroups < ngx) {
-                            const int64_t kn = gn < ngroups ? k0 + 32 * gn : kx + 32 * (gn - ngroups);
-#pragma unroll
-                            for (int i = 0; i < 2; i++) xg[sl][i] = *reinterpret_cast<const f32x4 *>(xp[i] + kn);
-                        }
+                        auto next_x = [&]() {
+                            constexpr int gn = gi + XD;
+                            if (gn < ngroups || gn - ngroups < ngx)
+                                fetch(xg[sl], gn < ngroups ? k0 + 32 * gn : kx + 32 * (gn - ngroups));
+                        };
+                        put_x(0);
+                        if (NT == 1) next_x();
                         if (gi == 0 && more) st.load(p, row0, rbase, N, pc + W, lane);
                         __builtin_amdgcn_wave_barrier();
                         Group<DT> g;
                         group_from_image<DT>(g, img, gi, d6);
                         float y[32];
                         g.decode(gi, y);
-                        tl.step(xs, lane, y);
+                        tl[0].step(xs, lane, y);
+                        if constexpr (NT == 2) {
+                            if (two) {
+                                put_x(1);
+                                __builtin_amdgcn_wave_barrier();
+                                tl[1].step(xs, lane, y);
+                            }
+                            next_x();
+                        }
                     }
                 });
                 __builtin_amdgcn_wave_barrier();
-                if (partial)
-                    tl.store_global(partial + (pc * M + m0) * N + rbase, N, mb, N - rbase, lane);
-                else
-                    tl.store(reinterpret_cast<float *>(ws), lane);
+#pragma unroll
+                for (int h = 0; h < NT; h++) {
+                    if (partial)
+                        tl[h].store_global(partial + (pc * M + m0 + 16 * h) * N + rbase, N, mb - 16 * h, N - rbase, lane);
+                    else
+                        tl[h].store(reinterpret_cast<float *>(ws) + 16 * h * kRPitch, lane);
+                }
             }
             if (!partial) {  // kernel-uniform
                 __syncthreads();
@@ -466,33 +488,99 @@ __global__ void sum_chunks_kernel(const float *__restrict__ partial, float *__re
 }
 
 
+// How a call is cut into workgroups: chunks of a row block in nslices slices of cps (1: a workgroup of kStageWaves covers
+// them all), passes of 16 or, two, 32 activation rows dealt over pz workgroups per row block and slice.
+struct RowsPlan {
+    int64_t nslices, cps, pz;
+    bool two;
+};
+
 template <int DT, int MT, int W>
 int run_tiles(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c, float *partial,
-              int64_t M, int64_t cps, int64_t nslices, bool acc) {
-    dim3 grid((unsigned)((N + 63) / 64), (unsigned)nslices), block(64 * W);
+              int64_t M, const RowsPlan &pl, bool acc) {
+    dim3 grid((unsigned)((N + 63) / 64), (unsigned)pl.nslices, (unsigned)pl.pz), block(64 * W);
     if (acc)
         hipLaunchKernelGGL((gemm_rows_mfma<DT, true, MT, W>), grid, block, 0, ctx->stream, w->planes(), x, c, partial, N,
-                           row0, M, w->K, cps);
+                           row0, M, w->K, pl.cps);
     else
         hipLaunchKernelGGL((gemm_rows_mfma<DT, false, MT, W>), grid, block, 0, ctx->stream, w->planes(), x, c, partial,
-                           N, row0, M, w->K, cps);
+                           N, row0, M, w->K, pl.cps);
     return launch_check(ctx, "gemm_rows");
 }
 
-// Up to 4 activation rows: one 4-row tile; up to 8: two; more: passes of 16 rows.
+// Up to 4 activation rows: one 4-row tile; up to 8: two; more: passes of 16 or 32 rows.
 template <int DT, int W>
 int run_w(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c, float *partial,
-          int64_t M, int64_t cps, int64_t nslices, bool acc) {
-    if (M <= 4) return run_tiles<DT, 1, W>(ctx, w, row0, N, x, c, partial, M, cps, nslices, acc);
-    if (M <= 8) return run_tiles<DT, 2, W>(ctx, w, row0, N, x, c, partial, M, cps, nslices, acc);
-    return run_tiles<DT, 0, W>(ctx, w, row0, N, x, c, partial, M, cps, nslices, acc);
+          int64_t M, const RowsPlan &pl, bool acc) {
+    if (M <= 4) return run_tiles<DT, 1, W>(ctx, w, row0, N, x, c, partial, M, pl, acc);
+    if (M <= 8) return run_tiles<DT, 2, W>(ctx, w, row0, N, x, c, partial, M, pl, acc);
+    if (pl.two) return run_tiles<DT, -1, W>(ctx, w, row0, N, x, c, partial, M, pl, acc);
+    return run_tiles<DT, 0, W>(ctx, w, row0, N, x, c, partial, M, pl, acc);
 }
 
 template <int DT>
 int run_dt(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c, float *partial,
-           int64_t M, int64_t cps, int64_t nslices, bool acc) {
-    if (partial) return run_w<DT, kSplitWaves>(ctx, w, row0, N, x, c, partial, M, cps, nslices, acc);
-    return run_w<DT, kStageWaves>(ctx, w, row0, N, x, c, partial, M, cps, nslices, acc);
+           int64_t M, const RowsPlan &pl, bool acc) {
+    if (partial) return run_w<DT, kSplitWaves>(ctx, w, row0, N, x, c, partial, M, pl, acc);
+    return run_w<DT, kStageWaves>(ctx, w, row0, N, x, c, partial, M, pl, acc);
+}
+
+// Up to 16 activation rows (one pass): one workgroup of kStageWaves waves per 64-row block covers all of its chunks when
+// there are enough row blocks to occupy the device; otherwise the chunks are split into slices of kSplitWaves chunks
+// (about two workgroups per CU in all) whose chain results are added in chunk order by sum_chunks_kernel.
+//
+// More rows: the plan of least estimated time. Registers and LDS hold two waves a SIMD, i.e. one workgroup of kStageWaves
+// or two of kSplitWaves a CU; so a plan takes ceil(workgroups / slots) rounds, a round the passes and chunk turns of one
+// workgroup. What a turn takes (two waves a SIMD; us for 16 rows and for 32, whose weights are decoded once) is measured
+// per format, in the larger workgroups with their sums in LDS and in the smaller ones; partial chain results cost a
+// launch, a write and a read. Passes dealt over workgroups instead of walked by one fill the device where row blocks are
+// few: 4096 x 4096, M = 77 (q4_k) 53 us walked, 41 in two workgroups per slice; 1024 x 4096, M = 300 172 walked, 50
+// dealt; 14336 x 4096, M = 512 862 walked in 16s, 655 dealt in 32s (784 dealt in 16s).
+struct TurnCost {
+    double whole[2], split[2];  // 16 rows, 32 rows
+};
+TurnCost turn_cost(int dtype) {
+    if (dtype == kQ8) return {{15.5, 31.0}, {18.0, 29.0}};
+    if (dtype == kQ6K) return {{18.0, 31.0}, {20.0, 33.0}};
+    return {{14.0, 24.0}, {12.5, 22.0}};
+}
+
+RowsPlan rows_plan(int dtype, int64_t M, int64_t N, int64_t nchunks, int64_t cus) {
+    const int64_t nrb = (N + 63) / 64;
+    RowsPlan split = {1, nchunks, 1, false};
+    if (nchunks > kSplitWaves) {
+        const int64_t want = (512 + nrb - 1) / nrb;  // slices per row block for about 512 workgroups
+        const int64_t maxs = (nchunks + kSplitWaves - 1) / kSplitWaves;
+        const int64_t ns = want < maxs ? want : maxs, cps = (nchunks + ns - 1) / ns;
+        split.cps = (cps + kSplitWaves - 1) / kSplitWaves * kSplitWaves;
+        split.nslices = (nchunks + split.cps - 1) / split.cps;
+    }
+    const RowsPlan whole = {1, nchunks, 1, false};
+    if (M <= 16) return nrb < 160 ? split : whole;
+    const TurnCost cost = turn_cost(dtype);
+    RowsPlan best = whole;
+    double least = 1e30;
+    for (int cut = 0; cut < (split.nslices > 1 ? 2 : 1); cut++)
+        for (int two = 0; two < 2; two++) {
+            RowsPlan p = cut ? split : whole;
+            p.two = two != 0;
+            const int64_t np = (M + (two ? 31 : 15)) / (two ? 32 : 16), waves = cut ? kSplitWaves : kStageWaves;
+            const int64_t slots = cus * (2 * 4 / waves), turns = (p.cps + waves - 1) / waves;
+            const double sums = cut ? 3.0 + (double)(nchunks * M * N) * 8.0 / 8e6 : 0.0;  // us, mostly cached
+            for (int64_t z = 1; z <= np && z <= 65535; z = z < 16 || z == np ? z + 1 : np) {
+                const int64_t wgs = nrb * p.nslices * z, rounds = (wgs + slots - 1) / slots, passes = (np + z - 1) / z;
+                const double alone = wgs * waves <= 4 * cus ? 0.82 : 1.0;  // one wave a SIMD
+                const double turn = alone * (cut ? cost.split[two] : cost.whole[two]);
+                // (a round's own start: its first weights and activations come from memory)
+                const double t = (double)rounds * ((double)(passes * turns) * turn + 4.0) + sums;
+                if (t < least) {
+                    least = t;
+                    p.pz = z;
+                    best = p;
+                }
+            }
+        }
+    return best;
 }
 
 }  // namespace
@@ -500,19 +588,9 @@ int run_dt(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const
 int launch_gemm_rows(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c,
                      int64_t M, bool acc) {
     if (N == 0 || M == 0) return TRHIP_OK;
-    const int64_t K = w->K, nchunks = (K + 255) / 256, nrb = (N + 63) / 64;
-    // One workgroup of kStageWaves waves per 64-row block covers all of its chunks when there are enough row blocks
-    // to occupy the device; otherwise the chunks are split into slices of kSplitWaves chunks (about two workgroups
-    // per CU in all) whose chain results are added in chunk order by sum_chunks_kernel.
-    int64_t nslices = 1, cps = nchunks;
-    if (nrb < 160 && nchunks > kSplitWaves) {
-        const int64_t want = (512 + nrb - 1) / nrb;  // slices per row block for about 512 workgroups
-        const int64_t maxs = (nchunks + kSplitWaves - 1) / kSplitWaves;
-        nslices = want < maxs ? want : maxs;
-        cps = (nchunks + nslices - 1) / nslices;
-        cps = (cps + kSplitWaves - 1) / kSplitWaves * kSplitWaves;
-        nslices = (nchunks + cps - 1) / cps;
-    }
+    const int64_t K = w->K, nchunks = (K + 255) / 256;
+    const RowsPlan pl = rows_plan(w->dtype, M, N, nchunks, ctx->sm_count > 0 ? ctx->sm_count : 256);
+    const int64_t nslices = pl.nslices;
     const bool copy_x = reinterpret_cast<uintptr_t>(x) % 16 != 0;  // the kernel reads x 16 bytes at a time
     const size_t xbytes = copy_x ? ((size_t)(M * K) * sizeof(float) + 255) / 256 * 256 : 0;
     const size_t pbytes = nslices > 1 ? (size_t)(nchunks * M * N) * sizeof(float) : 0;
@@ -530,10 +608,10 @@ int launch_gemm_rows(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_
     }
     float *partial = nslices > 1 ? reinterpret_cast<float *>(ws + xbytes) : nullptr;
     switch (w->dtype) {
-    case kQ8: st = run_dt<kQ8>(ctx, w, row0, N, xa, c, partial, M, cps, nslices, acc); break;
-    case kQ4: st = run_dt<kQ4>(ctx, w, row0, N, xa, c, partial, M, cps, nslices, acc); break;
-    case kQ4K: st = run_dt<kQ4K>(ctx, w, row0, N, xa, c, partial, M, cps, nslices, acc); break;
-    case kQ6K: st = run_dt<kQ6K>(ctx, w, row0, N, xa, c, partial, M, cps, nslices, acc); break;
+    case kQ8: st = run_dt<kQ8>(ctx, w, row0, N, xa, c, partial, M, pl, acc); break;
+    case kQ4: st = run_dt<kQ4>(ctx, w, row0, N, xa, c, partial, M, pl, acc); break;
+    case kQ4K: st = run_dt<kQ4K>(ctx, w, row0, N, xa, c, partial, M, pl, acc); break;
+    case kQ6K: st = run_dt<kQ6K>(ctx, w, row0, N, xa, c, partial, M, pl, acc); break;
     default: return fail(ctx, TRHIP_ERR_INVALID, "gemm_rows: bad dtype");
     }
     if (st != TRHIP_OK || !partial) return st;
