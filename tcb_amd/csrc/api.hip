@@ -946,6 +946,12 @@ int trhip_gemm_q_typed(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int6
             if (r != -1) return r;
         }
     }
+    // exact products of several rows of 16-bit x: the kernel widens x as it stages it and rounds c as it writes it. Two
+    // launches fewer: q4_k 1024x4096, M = 2, bf16 17.0 -> 12.8 us a call, q6_k 4096x14336, M = 3 43.8 -> 36.5
+    const uintptr_t xa = reinterpret_cast<uintptr_t>(x), ca = reinterpret_cast<uintptr_t>(c);
+    const bool apart = xa + 2 * (uintptr_t)(M * K) <= ca || ca + (uintptr_t)(M * N) * cb <= xa;  // c may not overwrite x
+    if (mode == TRHIP_MODE_EXACT && M > 1 && xtype != TRHIP_F32 && xa % 2 == 0 && ca % cb == 0 && apart)
+        return launch_gemm_rows(ctx, w, row0, N, x, c, M, accumulate != 0, xtype, ctype);
     // otherwise the reference's own sequence (gpu/backend_memory.go:41-52, 98-115): x widened to fp32, c widened when
     // accumulating, the fp32 operator, c rounded once
     const size_t xbytes = xtype == TRHIP_F32 ? 0 : (size_t)(M * K) * sizeof(float);

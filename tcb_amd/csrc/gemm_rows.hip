@@ -24,6 +24,7 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 // Plain vector types for registers carried across loop iterations (the HIP uint4 / float4 structs are copied with
 // memcpy, which keeps them in private memory there).
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -326,6 +327,28 @@ struct Tiles {
     }
 };
 
+// Element types of x and c (TRHIP_F32, or 16-bit ones widened exactly on use and rounded once; c is fp32 where x is), and
+// c (+)=.
+struct RowsIo {
+    int x, c;
+    bool acc;
+};
+__device__ __forceinline__ f32x4 widened(f32x4 v, int) { return v; }
+__device__ __forceinline__ f32x4 widened(u32x2 v, int io) {
+    return (f32x4){h16_to_f32(v.x & 0xFFFFu, io), h16_to_f32(v.x >> 16, io), h16_to_f32(v.y & 0xFFFFu, io),
+                   h16_to_f32(v.y >> 16, io)};
+}
+template <bool X16>
+__device__ __forceinline__ void put_c(void *c, int64_t i, float v, const RowsIo &io) {
+    if (!X16 || io.c == TRHIP_F32) {
+        float *o = static_cast<float *>(c) + i;
+        *o = io.acc ? *o + v : v;
+    } else {
+        uint16_t *o = static_cast<uint16_t *>(c) + i;
+        *o = (uint16_t)f32_to_h16(io.acc ? h16_to_f32(*o, io.c) + v : v, io.c);
+    }
+}
+
 // The same chains on the matrix cores, a pass of Tiles<MT>::kRows activation rows at a time, in ascending k from +0
 // as the CPU kernel does. Activation rows past M repeat row M - 1; their results are dropped.
 //
@@ -336,10 +359,13 @@ struct Tiles {
 // (loaded a few groups ahead) in a 16 x 32 LDS tile that its lanes read back as A operands. With partial == null
 // the workgroup covers every chunk and adds the chain results to `part` in chunk order in LDS; otherwise each
 // chain result goes to partial[chunk][m][row] for sum_chunks_kernel.
-template <int DT, bool ACC, int MT, int W>
-__global__ __launch_bounds__(64 * W) void gemm_rows_mfma(const Planes p, const float *__restrict__ x,
-                                                         float *__restrict__ c, float *__restrict__ partial, int64_t N,
-                                                         int64_t row0, int64_t M, int64_t K, int64_t cps) {
+template <int DT, bool X16, int MT, int W>
+__global__ __launch_bounds__(64 * W) void gemm_rows_mfma(const Planes p, const void *__restrict__ xv,
+                                                         void *__restrict__ c, float *__restrict__ partial, int64_t N,
+                                                         int64_t row0, int64_t M, int64_t K, int64_t cps, RowsIo io) {
+    using XT = std::conditional_t<X16, uint16_t, float>;
+    using XP = std::conditional_t<X16, u32x2, f32x4>;  // four activations as loaded
+    const XT *x = static_cast<const XT *>(xv);
     using I = Image<DT>;
     using TL = Tiles<MT < 0 ? 0 : MT>;
     constexpr int NT = MT < 0 ? 2 : 1, MP = NT * TL::kRows;  // tiles and activation rows of a pass
@@ -361,17 +387,17 @@ __global__ __launch_bounds__(64 * W) void gemm_rows_mfma(const Planes p, const f
     for (int64_t m0 = (int64_t)blockIdx.z * MP; m0 < M; m0 += (int64_t)gridDim.z * MP) {
         const int64_t mb = (M - m0) < MP ? (M - m0) : MP;
         const bool two = NT == 2 && mb > 16;  // the pass has rows for its second tile
-        const float *xp[2 * NT];  // x piece P = 64 i + lane: activation row P / 8, floats 4 (P % 8) .. +3 of a group
+        const XT *xp[2 * NT];  // x piece P = 64 i + lane: activation row P / 8, floats 4 (P % 8) .. +3 of a group
 #pragma unroll
         for (int i = 0; i < 2 * NT; i++) {
             const int P = 64 * i + lane, m = P >> 3;
             xp[i] = x + (m0 + (m < mb ? m : mb - 1)) * K + 4 * (P & 7);
         }
-        f32x4 xg[XD][2 * NT];  // activations of the next XD groups; group g of every chunk uses slot g % XD
-        auto fetch = [&](f32x4(&v)[2 * NT], int64_t k) {
+        XP xg[XD][2 * NT];  // activations of the next XD groups; group g of every chunk uses slot g % XD
+        auto fetch = [&](XP(&v)[2 * NT], int64_t k) {
 #pragma unroll
             for (int i = 0; i < 2 * NT; i++)
-                if (i < 2 || two) v[i] = *reinterpret_cast<const f32x4 *>(xp[i] + k);
+                if (i < 2 || two) v[i] = *reinterpret_cast<const XP *>(xp[i] + k);
         };
         constexpr int PR = 16 * NT / W;
         float part[PR];
@@ -408,7 +434,7 @@ __global__ __launch_bounds__(64 * W) void gemm_rows_mfma(const Planes p, const f
 #pragma unroll
                             for (int i = 0; i < 2; i++) {
                                 const int P = 64 * i + lane;
-                                *reinterpret_cast<f32x4 *>(xs + (P >> 3) * kXPitch + 4 * (P & 7)) = xg[sl][2 * h + i];
+                                *reinterpret_cast<f32x4 *>(xs + (P >> 3) * kXPitch + 4 * (P & 7)) = widened(xg[sl][2 * h + i], io.x);
                             }
                         };
                         // the activations XD groups on, then (once a chunk) the next chunk's weights, are in flight
@@ -461,18 +487,15 @@ __global__ __launch_bounds__(64 * W) void gemm_rows_mfma(const Planes p, const f
         if (!partial && r < N) {
 #pragma unroll
             for (int j = 0; j < PR; j++)
-                if (tm + W * j < mb) {
-                    float *o = c + (m0 + tm + W * j) * N + r;
-                    *o = ACC ? *o + part[j] : part[j];
-                }
+                if (tm + W * j < mb) put_c<X16>(c, (m0 + tm + W * j) * N + r, part[j], io);
         }
     }
 }
 
 // c[i] (+)= (((0 + partial[0][i]) + partial[1][i]) + ...) over the chunks in order, i < M N.
-template <bool ACC>
-__global__ void sum_chunks_kernel(const float *__restrict__ partial, float *__restrict__ c, int64_t MN,
-                                  int64_t nchunks) {
+template <bool X16>
+__global__ void sum_chunks_kernel(const float *__restrict__ partial, void *__restrict__ c, int64_t MN, int64_t nchunks,
+                                  RowsIo io) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < MN; i += (int64_t)gridDim.x * blockDim.x) {
         float part = 0.0f;
         for (int64_t ch = 0; ch < nchunks; ch += 8) {  // up to eight loads in flight, added in chunk order
@@ -483,7 +506,7 @@ __global__ void sum_chunks_kernel(const float *__restrict__ partial, float *__re
             for (int u = 0; u < 8; u++)
                 if (ch + u < nchunks) part = part + v[u];
         }
-        c[i] = ACC ? c[i] + part : part;
+        put_c<X16>(c, i, part, io);
     }
 }
 
@@ -495,34 +518,40 @@ struct RowsPlan {
     bool two;
 };
 
+struct RowsCall {
+    trhip_ctx *ctx;
+    const trhip_wstore *w;
+    int64_t row0, N, M;
+    const void *x;
+    void *c;
+    float *partial;
+    RowsPlan plan;
+    RowsIo io;
+};
+
 template <int DT, int MT, int W>
-int run_tiles(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c, float *partial,
-              int64_t M, const RowsPlan &pl, bool acc) {
-    dim3 grid((unsigned)((N + 63) / 64), (unsigned)pl.nslices, (unsigned)pl.pz), block(64 * W);
-    if (acc)
-        hipLaunchKernelGGL((gemm_rows_mfma<DT, true, MT, W>), grid, block, 0, ctx->stream, w->planes(), x, c, partial, N,
-                           row0, M, w->K, pl.cps);
-    else
-        hipLaunchKernelGGL((gemm_rows_mfma<DT, false, MT, W>), grid, block, 0, ctx->stream, w->planes(), x, c, partial,
-                           N, row0, M, w->K, pl.cps);
-    return launch_check(ctx, "gemm_rows");
+int run_tiles(const RowsCall &r) {
+    dim3 grid((unsigned)((r.N + 63) / 64), (unsigned)r.plan.nslices, (unsigned)r.plan.pz), block(64 * W);
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, grid, block, 0, r.ctx->stream, r.w->planes(), r.x, r.c, r.partial, r.N, r.row0, r.M,
+                           r.w->K, r.plan.cps, r.io);
+    };
+    if (r.io.x == TRHIP_F32) go(gemm_rows_mfma<DT, false, MT, W>);
+    else go(gemm_rows_mfma<DT, true, MT, W>);
+    return launch_check(r.ctx, "gemm_rows");
 }
 
 // Up to 4 activation rows: one 4-row tile; up to 8: two; more: passes of 16 or 32 rows.
 template <int DT, int W>
-int run_w(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c, float *partial,
-          int64_t M, const RowsPlan &pl, bool acc) {
-    if (M <= 4) return run_tiles<DT, 1, W>(ctx, w, row0, N, x, c, partial, M, pl, acc);
-    if (M <= 8) return run_tiles<DT, 2, W>(ctx, w, row0, N, x, c, partial, M, pl, acc);
-    if (pl.two) return run_tiles<DT, -1, W>(ctx, w, row0, N, x, c, partial, M, pl, acc);
-    return run_tiles<DT, 0, W>(ctx, w, row0, N, x, c, partial, M, pl, acc);
+int run_w(const RowsCall &r) {
+    if (r.M <= 4) return run_tiles<DT, 1, W>(r);
+    if (r.M <= 8) return run_tiles<DT, 2, W>(r);
+    return r.plan.two ? run_tiles<DT, -1, W>(r) : run_tiles<DT, 0, W>(r);
 }
 
 template <int DT>
-int run_dt(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c, float *partial,
-           int64_t M, const RowsPlan &pl, bool acc) {
-    if (partial) return run_w<DT, kSplitWaves>(ctx, w, row0, N, x, c, partial, M, pl, acc);
-    return run_w<DT, kStageWaves>(ctx, w, row0, N, x, c, partial, M, pl, acc);
+int run_dt(const RowsCall &r) {
+    return r.partial ? run_w<DT, kSplitWaves>(r) : run_w<DT, kStageWaves>(r);
 }
 
 // Up to 16 activation rows (one pass): one workgroup of kStageWaves waves per 64-row block covers all of its chunks when
@@ -540,7 +569,7 @@ struct TurnCost {
     double whole[2], split[2];  // 16 rows, 32 rows
 };
 TurnCost turn_cost(int dtype) {
-    if (dtype == kQ8) return {{15.5, 31.0}, {18.0, 29.0}};
+    if (dtype == kQ8) return {{15.9, 29.5}, {17.5, 29.0}};
     if (dtype == kQ6K) return {{18.0, 31.0}, {20.0, 33.0}};
     return {{14.0, 24.0}, {12.5, 22.0}};
 }
@@ -585,42 +614,44 @@ RowsPlan rows_plan(int dtype, int64_t M, int64_t N, int64_t nchunks, int64_t cus
 
 }  // namespace
 
-int launch_gemm_rows(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c,
-                     int64_t M, bool acc) {
+int launch_gemm_rows(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const void *x, void *c, int64_t M,
+                     bool acc, int xio, int cio) {
     if (N == 0 || M == 0) return TRHIP_OK;
     const int64_t K = w->K, nchunks = (K + 255) / 256;
     const RowsPlan pl = rows_plan(w->dtype, M, N, nchunks, ctx->sm_count > 0 ? ctx->sm_count : 256);
-    const int64_t nslices = pl.nslices;
-    const bool copy_x = reinterpret_cast<uintptr_t>(x) % 16 != 0;  // the kernel reads x 16 bytes at a time
-    const size_t xbytes = copy_x ? ((size_t)(M * K) * sizeof(float) + 255) / 256 * 256 : 0;
-    const size_t pbytes = nslices > 1 ? (size_t)(nchunks * M * N) * sizeof(float) : 0;
+    // the kernel reads x four elements at a time
+    const size_t xel = xio == TRHIP_F32 ? sizeof(float) : sizeof(uint16_t);
+    const bool copy_x = reinterpret_cast<uintptr_t>(x) % (4 * xel) != 0;
+    const size_t xbytes = copy_x ? ((size_t)(M * K) * xel + 255) / 256 * 256 : 0;
+    const size_t pbytes = pl.nslices > 1 ? (size_t)(nchunks * M * N) * sizeof(float) : 0;
     int st = TRHIP_OK;
     uint8_t *ws = nullptr;
     if (xbytes + pbytes > 0) {
         ws = static_cast<uint8_t *>(workspace(ctx, xbytes + pbytes, &st));
         if (!ws) return st;
     }
-    const float *xa = x;
+    RowsCall r = {ctx, w, row0, N, M, x, c, nullptr, pl, {xio, cio, acc}};
     if (copy_x) {
-        hipError_t e = hipMemcpyAsync(ws, x, (size_t)(M * K) * sizeof(float), hipMemcpyDeviceToDevice, ctx->stream);
+        hipError_t e = hipMemcpyAsync(ws, x, (size_t)(M * K) * xel, hipMemcpyDeviceToDevice, ctx->stream);
         if (e != hipSuccess) return hip_fail(ctx, e, "gemm_rows: align x");
-        xa = reinterpret_cast<const float *>(ws);
+        r.x = ws;
     }
-    float *partial = nslices > 1 ? reinterpret_cast<float *>(ws + xbytes) : nullptr;
+    if (pl.nslices > 1) r.partial = reinterpret_cast<float *>(ws + xbytes);
     switch (w->dtype) {
-    case kQ8: st = run_dt<kQ8>(ctx, w, row0, N, xa, c, partial, M, pl, acc); break;
-    case kQ4: st = run_dt<kQ4>(ctx, w, row0, N, xa, c, partial, M, pl, acc); break;
-    case kQ4K: st = run_dt<kQ4K>(ctx, w, row0, N, xa, c, partial, M, pl, acc); break;
-    case kQ6K: st = run_dt<kQ6K>(ctx, w, row0, N, xa, c, partial, M, pl, acc); break;
+    case kQ8: st = run_dt<kQ8>(r); break;
+    case kQ4: st = run_dt<kQ4>(r); break;
+    case kQ4K: st = run_dt<kQ4K>(r); break;
+    case kQ6K: st = run_dt<kQ6K>(r); break;
     default: return fail(ctx, TRHIP_ERR_INVALID, "gemm_rows: bad dtype");
     }
-    if (st != TRHIP_OK || !partial) return st;
+    if (st != TRHIP_OK || !r.partial) return st;
     const int64_t MN = M * N;
     const unsigned blocks = (unsigned)((MN + 255) / 256 < 4096 ? (MN + 255) / 256 : 4096);
-    if (acc)
-        hipLaunchKernelGGL(sum_chunks_kernel<true>, dim3(blocks), dim3(256), 0, ctx->stream, partial, c, MN, nchunks);
-    else
-        hipLaunchKernelGGL(sum_chunks_kernel<false>, dim3(blocks), dim3(256), 0, ctx->stream, partial, c, MN, nchunks);
+    auto sum = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, ctx->stream, r.partial, c, MN, nchunks, r.io);
+    };
+    if (xio == TRHIP_F32) sum(sum_chunks_kernel<false>);
+    else sum(sum_chunks_kernel<true>);
     return launch_check(ctx, "sum_chunks");
 }
 

@@ -411,8 +411,9 @@ int launch_gemv(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, 
 // bit-identical to the fast GEMV followed by launch_swiglu. Returns -1 (nothing launched) where the fused kernel
 // does not apply.
 int launch_gemv_fast_swiglu(trhip_ctx *ctx, const trhip_wstore *w, const float *x, float *out, int64_t I);
-int launch_gemm_rows(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c,
-                     int64_t M, bool acc);
+// xio, cio: element types of x and c (TRHIP_F32, TRHIP_F16, TRHIP_BF16), cio fp32 where xio is; aligned to their size
+int launch_gemm_rows(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const void *x, void *c, int64_t M,
+                     bool acc, int xio = TRHIP_F32, int cio = TRHIP_F32);
 // swi != nullptr (set, not accumulate; N = 2I rows [gate | up]): out swi[m, i] = silu(c[m, i]) * c[m, I + i], fused
 // into the slice sum when K is split (c is then not written), else after it
 int launch_gemm_rows_fast(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c,

@@ -6,7 +6,7 @@ import pytest
 
 import oracle as O
 from conftest import same_bits
-from tcb_amd import Q4, Q4K, Q6K, Q8, synth
+from tcb_amd import BF16, F16, F32, MODE_EXACT, Q4, Q4K, Q6K, Q8, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -38,5 +38,33 @@ def test_rows_plan_bits(backend, dt, M, N, K):
     assert np.array_equal(np.isnan(got[M - 1]), np.isnan(want[-1]))
     assert np.isfinite(got[:M - 1]).all()
     for b in (xb, cb):
+        b.free()
+    w.release()
+
+
+@pytest.mark.parametrize("xt,ct", [(F16, F16), (BF16, BF16), (F32, F16), (BF16, F32)])
+@pytest.mark.parametrize("dt,M,N,K,off", [(Q8, 2, 300, 4096, 0), (Q4K, 6, 130, 2048, 2), (Q6K, 13, 64, 512, 6),
+                                          (Q4, 40, 200, 2560, 0), (Q4K, 33, 10300, 256, 0)])
+def test_rows_typed_bits(backend, xt, ct, dt, M, N, K, off):
+    """16-bit x widened as it is staged and 16-bit c rounded as it is written (by the product or by the sum of its
+    slices), x off the kernel's alignment included: the bits of the fp32 call on the widened activations, rounded."""
+    raw = synth.quant_weights(dt, N, K, seed=N + K, outliers=0.01)
+    w = backend.FromQuantized(dt, raw, N, K)
+    x, c0 = synth.activations(M, K, seed=K + M).reshape(-1), synth.activations(M, N, seed=N).reshape(-1)
+    x[K + 1], c0[5] = np.nan, np.inf
+    xa = x if xt == F32 else O.round16(xt, x)
+    ca = c0 if ct == F32 else O.round16(ct, c0)
+    xw, cw = x if xt == F32 else O.widen16(xt, xa), c0 if ct == F32 else O.widen16(ct, ca)
+    off *= 2 if xt == F32 else 1
+    xb = backend.ctx.alloc(xa.nbytes + 64)
+    xb.upload(xa, byte_offset=off)
+    cb, x32, c32 = backend.ctx.to_device(ca), backend.ctx.to_device(xw), backend.ctx.to_device(cw)
+    backend.GemmTyped(M, N, K, (xb, off), xt, w, cb, ct, accumulate=True, mode=MODE_EXACT)
+    backend.Gemm(M, N, K, x32, w, c32)
+    got, want = cb.download(np.float32 if ct == F32 else np.uint16, M * N), c32.download(np.float32, M * N)
+    if ct != F32:
+        got, want = O.widen16(ct, got), O.widen16(ct, O.round16(ct, want))
+    same_bits(got, want)
+    for b in (xb, cb, x32, c32):
         b.free()
     w.release()
