@@ -144,9 +144,9 @@ int trhip_wstore_to_raw(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int
  * M == 1 GEMV of every dtype on fixed-point activations (K up to 16384; q8_0 / q4_0 with an even
  * block count), q4_k with 5 <= M <= 16 on f16 matrix cores over two-term activations and with M > 16
  * on int8 matrix cores, q4_0 with 2 <= M <= 16 (K a multiple of 256) and q6_k with M > 1 on f16 matrix
- * cores, and large products (M > 16) of every dtype on f16 matrix cores over two-term activations; other
- * cases run exact. The reference GPU's GEMV and its M > 1 dequantize-and-GEMM are tolerance-bound too
- * (gpu/kernel_quant_gemv.go:33-84, gpu/backend_quant.go:43-134). */
+ * cores, and large products (M > 16) of every dtype on 16-bit matrix cores: q8_0 and q4_0 over three bf16
+ * terms that hold x exactly, the k-quants over two f16 terms; other cases run exact. The reference GPU's GEMV and its
+ * M > 1 dequantize-and-GEMM are tolerance-bound too (gpu/kernel_quant_gemv.go:33-84, gpu/backend_quant.go:43-134). */
 int trhip_gemm_q(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x,
                  float *c, int64_t M, int64_t K, int accumulate, int mode);
 

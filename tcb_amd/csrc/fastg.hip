@@ -1,20 +1,25 @@
-// fastg.hip -- fast-mode (tolerance) product of fp32 activations for more than 16 rows, every weight format, on f16
+// fastg.hip -- fast-mode (tolerance) product of fp32 activations for more than 16 rows, every weight format, on 16-bit
 // matrix cores: trhip_gemm_q(TRHIP_MODE_FAST). The reference's GPU runs these as dequantized tiles through a float GEMM
 // (gpu/backend_quant.go:43-134), a tolerance path too.
 //
-// Activations: each row is scaled by a power of two, x' = x 2^(14 - E) with 2^E > max|x| of the row, and split into two
-// f16 terms, hi = f16(x') and lo = f16(x' - hi): exact to 2^-23 of each element, and to 2^-39 of the row's largest where
-// lo is subnormal (the f16 MFMAs keep subnormals). Weights: the integer part of every format is exact in f16,
+// Activations: each row is scaled by a power of two, x' = x 2^(14 - E) with 2^E > max|x| of the row, and split.
+//   q8_0, q4_0: three bf16 terms of eight bits, which add up to x' exactly, whatever the range of the row (bf16 has fp32's
+//     exponents; elements below 2^-110 of the row's largest lose low bits). Two f16 terms, exact to 2^-39 of the row's
+//     largest only, were 10-25% faster (4096 x 14336, M = 300 134 against 164 us) and lost every element beside one 2^40
+//     times larger.
+//   q4_k, q6_k: two f16 terms, hi = f16(x') and lo = f16(x' - hi): exact to 2^-23 of each element, and to 2^-39 of the
+//     row's largest where lo is subnormal (the f16 MFMAs keep subnormals).
+// Weights: the integer part of every format is exact in the terms' type,
 //   q8_0, q4_0: the code (q4 - 8);   q4_k: q4 sc - o;   q6_k: (q6 - 32) (sc & ~1) and (q6 - 32) (sc & 1), two planes
 // so each product is exact and only fp32 sums round. Per block (32 elements for q8_0 and q4_0, 256 for the k-quants)
-//   acc += d D,   D = sum w (hi + lo);   q4_k: acc += d D + sum_j v_j S_j,   v_j = d o_j - dmin m_j
+//   acc += d D,   D = sum w x'   (over the terms);   q4_k: acc += d D + sum_j v_j S_j,   v_j = d o_j - dmin m_j
 // with S_j the sub-block sums of x' as three f16 terms and v_j, scaled by a power of two per block, as two. o_j is an
 // integer near dmin m_j / d, so that the code and minimum terms, several times the result, cancel in no sum. (Error
 // against float64 at K = 4096: 1.5e-7; with o_j = 8 sc_j 3.0e-7; the exact mode's 3.0e-7, the int8 digits' 2.2e-7.)
 //
 // Tiles. A workgroup is 8 waves over 32 WM activation rows and 256 weight rows. The weights of 64 elements are expanded
 // once per workgroup, by all threads, into LDS in operand order (two buffers, one barrier per 64 elements); a wave
-// multiplies 32 activation rows by 32 CT of the columns, so each B operand read from LDS serves two MFMAs (hi, lo) and
+// multiplies 32 activation rows by 32 CT of the columns, so each B operand read from LDS serves an MFMA per term and
 // each A operand, read straight from the split activations in L2, CT of them. (Weights expanded into each wave's own
 // registers would leave an A operand one MFMA at 32 columns a wave, and the A reads alone would fill the LDS bandwidth.)
 //
@@ -23,7 +28,7 @@
 // than 87 us; the kernel with its operand reads, expansion and folding taken out took 90, each of them adds its own time
 // (A reads 17 us, expansion 27, folding 12), whether the two waves of a SIMD work in step or in opposite phases: 144 us a
 // call (digits kernel 195). Multiplying before expanding, in each step, measured 143.8 against 152.6 us. q8_0 (exact
-// K = 1 products before): 14336 x 4096, M = 512 996 -> 150; 4096 x 14336, M = 300 722 -> 128.
+// K = 1 products before): 14336 x 4096, M = 300 606 -> 185; 4096 x 14336, M = 300 725 -> 164.
 #include "trhip_internal.hpp"
 #include "mfma_util.hpp"
 
@@ -33,13 +38,31 @@ namespace trhip {
 namespace {
 
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef __bf16 v8b __attribute__((ext_vector_type(8)));
 
 constexpr int FG_W = 8, FG_THREADS = 64 * FG_W, FG_TN = 256;
 constexpr int FG_E = 14;  // |x'| < 2^14
 
+template <int DT>
+struct Fg {
+    static constexpr bool KQ = DT == kQ4K || DT == kQ6K;
+    static constexpr int TERMS = KQ ? 2 : 3;                  // of an activation
+    static constexpr int PL = DT == kQ6K ? 2 : 1;             // planes per weight
+    static constexpr int B = PL * 4 * 8 * 1024;               // operands of a step: [plane][step][column tile][lane][16]
+    static constexpr int DS = KQ ? 0 : 2 * FG_TN * 4;         // d of the step's two blocks
+    static constexpr int BUF = B + DS;
+    static constexpr int CO = DT == kQ4K ? FG_TN * 64 : 0;     // q4_k: v_j 2^-q as two f16 terms; the code constants
+    static constexpr int DK = KQ ? FG_TN * 8 : 0;             // per column d and (q4_k) 2^(q + 6), S_j being scaled 2^-6
+    static constexpr int BLK = CO + DK;                       // per block, two buffers
+    static constexpr size_t LDS = 2 * BUF + 2 * BLK;
+};
+static_assert(Fg<kQ6K>::LDS <= 160 * 1024 && Fg<kQ4K>::LDS <= 160 * 1024, "one workgroup per CU");
+
 // ---- activations ----
 
-// Largest |x| of each 1024-element piece of a row (pm[m][piece], infinity if it holds NaN / Inf). One wave a piece.
+// Largest |x| of each 1024-element piece of a row, one wave a piece: pm[m][piece], infinity if it holds NaN / Inf
+// (k-quants); FINITE (q8_0, q4_0): of its finite elements.
+template <bool FINITE>
 __global__ __launch_bounds__(256) void row_max_kernel(const float *__restrict__ x, int64_t M, int64_t K, int64_t np,
                                                       float *__restrict__ pm) {
     const int lane = threadIdx.x & 63;
@@ -52,7 +75,13 @@ __global__ __launch_bounds__(256) void row_max_kernel(const float *__restrict__ 
     for (int i = 0; i < 4; i++) {
         const int64_t k = k0 + 256 * i + 4 * lane;
         const float4 v = *reinterpret_cast<const float4 *>(x + m * K + (k < K ? k : 0));
-        if (k < K) {
+        if (k >= K) continue;
+        if (FINITE) {
+            const float e[4] = {fabsf(v.x), fabsf(v.y), fabsf(v.z), fabsf(v.w)};
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (e[j] <= FLT_MAX) a = fmaxf(a, e[j]);
+        } else {
             a = fmaxf(a, amax4(v));
             bad |= non_finite4(v) != 0;
         }
@@ -63,15 +92,19 @@ __global__ __launch_bounds__(256) void row_max_kernel(const float *__restrict__ 
     if (lane == 0) pm[t] = bad ? __builtin_inff() : a;
 }
 
-// The split activations: per 32-row tile and 16-element step, 1 KB of hi operands and 1 KB of lo (lane r + 32 h: row r,
-// elements 8 h .. + 7 of the step, each four as 0, 2, 1, 3: the order in which nibbles and bytes pair up in a dword).
+// The split activations: per 32-row tile and 16-element step, 1 KB of operands of each term, largest term first (lane
+// r + 32 h: row r, elements 8 h .. + 7 of the step, each four as 0, 2, 1, 3: the order in which nibbles and bytes pair up
+// in a dword). q8_0 / q4_0: three bf16 terms cut off x' in turn, eight bits each, so that they add up to x' exactly; a NaN
+// or Inf is its first term.
 // K is padded with zeros to a multiple of 64, rows to 32. q4_k: the sub-block sums S_j 2^-6 as three f16 terms, per tile
 // and 256-element block two operands [P0 | P1], [P0 | P2] (times [vh | vh], [vl | vh] of the weights). Workgroup (tile, 256-element chunk); ex[m] = E - 14, bad[m].
-template <bool SUMS>
+template <int DT>
 __global__ __launch_bounds__(256) void split_kernel(const float *__restrict__ x, int64_t M, int64_t K, int64_t np,
                                                     const float *__restrict__ pm, uint8_t *__restrict__ rec,
                                                     uint8_t *__restrict__ srec, int *__restrict__ ex,
                                                     int *__restrict__ bad) {
+    constexpr bool SUMS = DT == kQ4K;
+    constexpr int TERMS = Fg<DT>::TERMS;
     const int tid = threadIdx.x, r = tid >> 3, s8 = tid & 7;
     const int64_t nch = (K + 255) / 256, mt = blockIdx.x / nch, ch = blockIdx.x % nch;
     const int64_t m = 32 * mt + r, KS = (K + 63) / 64 * 4;
@@ -85,7 +118,7 @@ __global__ __launch_bounds__(256) void split_kernel(const float *__restrict__ x,
     if (!inf && a > 0.0f) (void)frexpf(a, &E);
     if (ch == 0 && s8 == 0 && row) {
         ex[m] = E - FG_E;
-        bad[m] = inf ? 1 : 0;
+        if (Fg<DT>::KQ) bad[m] = inf ? 1 : 0;
     }
     const bool use = row && !inf;
 #pragma unroll
@@ -97,23 +130,36 @@ __global__ __launch_bounds__(256) void split_kernel(const float *__restrict__ x,
         const float4 *p = reinterpret_cast<const float4 *>(x + (in ? m * K + k : 0));
         const float4 v0 = p[0], v1 = p[1];
         const float raw[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-        uint16_t hi[8], lo[8];
+        uint16_t tm[TERMS][8];
         double s = 0.0;
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             v[i] = in ? ldexpf(raw[i], FG_E - E) : 0.0f;
-            const _Float16 h = (_Float16)v[i];
-            hi[i] = __builtin_bit_cast(uint16_t, h);
-            lo[i] = __builtin_bit_cast(uint16_t, (_Float16)(v[i] - (float)h));
+            if constexpr (TERMS == 3) {
+                const uint32_t u = __builtin_bit_cast(uint32_t, v[i]);
+                const bool fin = (u & 0x7F800000u) != 0x7F800000u;
+                float rest = v[i];
+#pragma unroll
+                for (int t = 0; t < 3; t++) {
+                    const uint32_t top = __builtin_bit_cast(uint32_t, rest) & 0xFFFF0000u;
+                    tm[t][i] = (uint16_t)(top >> 16);
+                    rest = fin ? rest - __builtin_bit_cast(float, top) : 0.0f;
+                }
+                if (!fin && (u & 0x007FFFFFu)) tm[0][i] |= 0x40;  // a NaN whose payload is all in the cut bits
+            } else {
+                const _Float16 h = (_Float16)v[i];
+                tm[0][i] = __builtin_bit_cast(uint16_t, h);
+                tm[1][i] = __builtin_bit_cast(uint16_t, (_Float16)(v[i] - (float)h));
+            }
             if (SUMS) s += (double)v[i];
         }
         auto pack = [](const uint16_t (&u)[8]) {
             return make_uint4(u[0] | (uint32_t)u[2] << 16, u[1] | (uint32_t)u[3] << 16, u[4] | (uint32_t)u[6] << 16,
                               u[5] | (uint32_t)u[7] << 16);
         };
-        uint8_t *o = rec + ((mt * KS + (k >> 4)) * 2) * 1024 + (r + 32 * (s8 & 1)) * 16;
-        *reinterpret_cast<uint4 *>(o) = pack(hi);
-        *reinterpret_cast<uint4 *>(o + 1024) = pack(lo);
+        uint8_t *o = rec + ((mt * KS + (k >> 4)) * TERMS) * 1024 + (r + 32 * (s8 & 1)) * 16;
+#pragma unroll
+        for (int t = 0; t < TERMS; t++) *reinterpret_cast<uint4 *>(o + 1024 * t) = pack(tm[t]);
         if (SUMS) {
             s += __shfl_xor(s, 1);
             s += __shfl_xor(s, 2);
@@ -147,6 +193,16 @@ __device__ __forceinline__ h2 pair_f16(uint32_t w, uint32_t mask, uint32_t k64, 
 }
 __device__ __forceinline__ uint32_t bits(h2 v) { return __builtin_bit_cast(uint32_t, v); }
 
+// The four signed bytes of a dword as bf16 pairs, bytes 0, 2 and 1, 3: the upper halves of the integers' fp32 values, which
+// hold them exactly (eight significant bits).
+__device__ __forceinline__ void bytes4(uint32_t w, uint32_t &p02, uint32_t &p13) {
+    uint32_t f[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) f[i] = __builtin_bit_cast(uint32_t, (float)(int8_t)(w >> (8 * i)));
+    p02 = __builtin_amdgcn_perm(f[2], f[0], 0x07060302u);
+    p13 = __builtin_amdgcn_perm(f[3], f[1], 0x07060302u);
+}
+
 // (1024 + 16 q) m + a for the eight nibbles q of a dword, each at bits 4..7 of a half word: with m = s / 16 and an integer
 // a near -64 s this is q s + 64 s + a, exactly. The pairs are bytes 0, 2 and 1, 3.
 __device__ __forceinline__ void nibbles8(uint32_t w, uint32_t k64, _Float16 ml, _Float16 al, _Float16 mh, _Float16 ah,
@@ -156,20 +212,6 @@ __device__ __forceinline__ void nibbles8(uint32_t w, uint32_t k64, _Float16 ml, 
     hi[0] = bits(pair_f16(w, 0x00F000F0u, k64, mh, ah));
     hi[1] = bits(pair_f16(w >> 8, 0x00F000F0u, k64, mh, ah));
 }
-
-template <int DT>
-struct Fg {
-    static constexpr bool KQ = DT == kQ4K || DT == kQ6K;
-    static constexpr int PL = DT == kQ6K ? 2 : 1;             // f16 planes per weight
-    static constexpr int B = PL * 4 * 8 * 1024;               // operands of a step: [plane][step][column tile][lane][16]
-    static constexpr int DS = KQ ? 0 : 2 * FG_TN * 4;         // d of the step's two blocks
-    static constexpr int BUF = B + DS;
-    static constexpr int CO = DT == kQ4K ? FG_TN * 64 : 0;     // q4_k: v_j 2^-q as two f16 terms; the code constants
-    static constexpr int DK = KQ ? FG_TN * 8 : 0;             // per column d and (q4_k) 2^(q + 6), S_j being scaled 2^-6
-    static constexpr int BLK = CO + DK;                       // per block, two buffers
-    static constexpr size_t LDS = 2 * BUF + 2 * BLK;
-};
-static_assert(Fg<kQ6K>::LDS <= 160 * 1024 && Fg<kQ4K>::LDS <= 160 * 1024, "one workgroup per CU");
 
 template <int DT>
 struct ColW;
@@ -187,19 +229,14 @@ struct ColW<kQ8> {
         a[i][1] = q[1];
         d[i] = p.d[b];
     }
-    __device__ __forceinline__ void expand(uint8_t *buf, int c, int h, int i, uint32_t k64) {
+    __device__ __forceinline__ void expand(uint8_t *buf, int c, int h, int i) {
         uint8_t *o = buf + ((2 * h) * 8 + (c >> 5)) * 1024 + (c & 31) * 16;
 #pragma unroll
         for (int ks = 0; ks < 2; ks++) {
             const uint32_t w[4] = {a[i][ks].x, a[i][ks].y, a[i][ks].z, a[i][ks].w};
             uint32_t v[8];
 #pragma unroll
-            for (int e = 0; e < 4; e++) {  // signed bytes as q + 128: (1024 + q + 128) - 1152
-                const uint32_t u = w[e] ^ 0x80808080u;
-                const h2 off = (h2){(_Float16)-1152.0f, (_Float16)-1152.0f};
-                v[2 * e] = bits(__builtin_bit_cast(h2, __builtin_amdgcn_perm(k64, u, 0x05020500u)) + off);
-                v[2 * e + 1] = bits(__builtin_bit_cast(h2, __builtin_amdgcn_perm(k64, u, 0x05030501u)) + off);
-            }
+            for (int e = 0; e < 4; e++) bytes4(w[e], v[2 * e], v[2 * e + 1]);
             *reinterpret_cast<uint4 *>(o + ks * 8192) = make_uint4(v[0], v[1], v[2], v[3]);
             *reinterpret_cast<uint4 *>(o + ks * 8192 + 512) = make_uint4(v[4], v[5], v[6], v[7]);
         }
@@ -217,14 +254,16 @@ struct ColW<kQ4> {
         a[i] = *reinterpret_cast<const uint4 *>(p.qs + b * 16);
         d[i] = p.d[b];
     }
-    __device__ __forceinline__ void expand(uint8_t *buf, int c, int h, int i, uint32_t k64) {
+    __device__ __forceinline__ void expand(uint8_t *buf, int c, int h, int i) {
         // byte j holds elements j (low nibble, operand step 2 h) and j + 16 (high, step 2 h + 1)
         uint8_t *o = buf + ((2 * h) * 8 + (c >> 5)) * 1024 + (c & 31) * 16;
         const uint32_t w[4] = {a[i].x, a[i].y, a[i].z, a[i].w};
         uint32_t lo[4][2], hi[4][2];
 #pragma unroll
-        for (int e = 0; e < 4; e++)
-            nibbles8(w[e], k64, (_Float16)0.0625f, (_Float16)-72.0f, (_Float16)0.0625f, (_Float16)-72.0f, lo[e], hi[e]);
+        for (int e = 0; e < 4; e++) {  // q - 8 as signed bytes: (q + 120) ^ 128, no carry between bytes
+            bytes4(((w[e] & 0x0F0F0F0Fu) + 0x78787878u) ^ 0x80808080u, lo[e][0], lo[e][1]);
+            bytes4((((w[e] >> 4) & 0x0F0F0F0Fu) + 0x78787878u) ^ 0x80808080u, hi[e][0], hi[e][1]);
+        }
         *reinterpret_cast<uint4 *>(o) = make_uint4(lo[0][0], lo[0][1], lo[1][0], lo[1][1]);
         *reinterpret_cast<uint4 *>(o + 512) = make_uint4(lo[2][0], lo[2][1], lo[3][0], lo[3][1]);
         *reinterpret_cast<uint4 *>(o + 8192) = make_uint4(hi[0][0], hi[0][1], hi[1][0], hi[1][1]);
@@ -354,7 +393,7 @@ __global__ __launch_bounds__(FG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
     const int *__restrict__ bad, int64_t cps, float *__restrict__ c, float *__restrict__ partial, int acc_c) {
     using L = Fg<DT>;
     constexpr bool KQ = L::KQ;
-    constexpr int TM = 32 * WM, PL = L::PL;
+    constexpr int TM = 32 * WM, PL = L::PL, TERMS = L::TERMS;
     static_assert(FG_W / WM * CT * 32 == FG_TN, "the waves cover the tile");
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -369,14 +408,14 @@ __global__ __launch_bounds__(FG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
     const int64_t wrow = row0 + (n0 + col < N ? n0 + col : N - 1);
     auto bufp = [&](int i) { return lds + i * L::BUF; };
     auto blkp = [&](int i) { return lds + 2 * L::BUF + i * L::BLK; };
-    const uint8_t *arec = rec + mt * (4 * (int64_t)ns) * 2048;  // wave-uniform
+    const uint8_t *arec = rec + mt * (4 * (int64_t)ns) * (TERMS * 1024);  // wave-uniform
     const uint32_t l16 = 16 * (uint32_t)lane;
     auto clamp_s = [&](int s) { return s < ns ? s : ns - 1; };
     auto clamp_c = [&](int ch) { return ch < nch ? ch : nch - 1; };
 
     const uint32_t k64 = hide(0x64006400u);
     ColW<DT> W;
-    v8h A[4][2];
+    v8h A[4][TERMS];
     if constexpr (KQ) {
 #pragma unroll
         for (int g = 0; g < 4; g++) W.load(p, wrow, ch0, h, g);
@@ -391,13 +430,14 @@ __global__ __launch_bounds__(FG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
     } else {
         W.load(p, wrow, 4 * ch0, h, 0);
         W.load(p, wrow, clamp_s(4 * ch0 + 1), h, 1);
-        W.expand(bufp(0), col, h, 0, k64);
+        W.expand(bufp(0), col, h, 0);
         W.load(p, wrow, clamp_s(4 * ch0 + 2), h, 0);
     }
 #pragma unroll
     for (int ks = 0; ks < 4; ks++)
 #pragma unroll
-        for (int t = 0; t < 2; t++) A[ks][t] = *reinterpret_cast<const v8h *>(arec + (int64_t)(32 * ch0 + 2 * ks + t) * 1024 + l16);
+        for (int t = 0; t < TERMS; t++)
+            A[ks][t] = *reinterpret_cast<const v8h *>(arec + (int64_t)((16 * ch0 + ks) * TERMS + t) * 1024 + l16);
 
     float acc[CT][16];
 #pragma unroll
@@ -407,9 +447,9 @@ __global__ __launch_bounds__(FG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
     v16f D[KQ ? CT : 1];
     // the registers of operand step ks are refilled with the next step's as soon as they have been multiplied
     auto refill = [&](int ks, int s) {
-        const uint8_t *an = arec + (int64_t)(8 * clamp_s(s + 1) + 2 * ks) * 1024;
-        A[ks][0] = *reinterpret_cast<const v8h *>(an + l16);
-        A[ks][1] = *reinterpret_cast<const v8h *>(an + 1024 + l16);
+        const uint8_t *an = arec + (int64_t)((4 * clamp_s(s + 1) + ks) * TERMS) * 1024;
+#pragma unroll
+        for (int t = 0; t < TERMS; t++) A[ks][t] = *reinterpret_cast<const v8h *>(an + 1024 * t + l16);
     };
 
     // Fold block ch (k-quants) into the sums.
@@ -486,10 +526,11 @@ __global__ __launch_bounds__(FG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
                     dv[i & 1] = ds[FG_TN * blk + 32 * t];
                     v16f e = (v16f){0.0f};
 #pragma unroll
-                    for (int k = 0; k < 2; k++)
+                    for (int q = TERMS - 1; q >= 0; q--)  // small terms first
 #pragma unroll
-                        for (int q = 0; q < 2; q++)
-                            e = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[2 * blk + k][q], B[i & 1][k], e, 0, 0, 0);
+                        for (int k = 0; k < 2; k++)
+                            e = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8b, A[2 * blk + k][q]),
+                                                                        __builtin_bit_cast(v8b, B[i & 1][k]), e, 0, 0, 0);
                     E[i & 1] = e;
                     if (t == CT - 1) {
                         refill(2 * blk, s);
@@ -520,7 +561,7 @@ __global__ __launch_bounds__(FG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
                         for (int q = 0; q < 4; q++) W.load(p, wrow, clamp_c(ch + 1), h, q);
                     }
                 } else {
-                    W.expand(nb, col, h, (g + 1) & 1, k64);
+                    W.expand(nb, col, h, (g + 1) & 1);
                     W.load(p, wrow, clamp_s(s + 3), h, (g + 1) & 1);
                 }
             }
@@ -534,7 +575,7 @@ __global__ __launch_bounds__(FG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
     for (int v = 0; v < 16; v++) {
         const int64_t m = m0 + 32 * wm + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
         const int e = ex[m < M ? m : M - 1];
-        const bool ok = m < M && !bad[m < M ? m : M - 1];
+        const bool ok = m < M && (!KQ || !bad[m < M ? m : M - 1]);
 #pragma unroll
         for (int t = 0; t < CT; t++) {
             const int64_t n = n0 + 32 * (CT * wn + t) + (lane & 31);
@@ -545,6 +586,7 @@ __global__ __launch_bounds__(FG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
             }
         }
     }
+    if constexpr (!KQ) return;  // (NaN and Inf are ordinary terms there)
     // rows holding NaN/Inf: exact float dot products (in the first slice; the others add +0); rare
     if (!__syncthreads_or(tid < TM && m0 + tid < M && bad[m0 + tid])) return;
     for (int i = tid; i < TM * FG_TN; i += FG_THREADS) {
@@ -630,7 +672,8 @@ int launch_fast_gemm(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_
     nsl = (nch + cps - 1) / cps;
     auto al = [](size_t v) { return (v + 255) / 256 * 256; };
     const bool copy_x = reinterpret_cast<uintptr_t>(x) % 16 != 0;
-    const size_t o_s = al((size_t)(mt * KS) * 2048), o_pm = al(o_s + (w->dtype == kQ4K ? (size_t)(mt * nch) * 2048 : 0));
+    const bool kq = w->dtype == kQ4K || w->dtype == kQ6K;
+    const size_t o_s = al((size_t)(mt * KS) * (kq ? 2048 : 3072)), o_pm = al(o_s + (w->dtype == kQ4K ? (size_t)(mt * nch) * 2048 : 0));
     const size_t o_ex = al(o_pm + (size_t)(M * np) * sizeof(float)), o_bad = al(o_ex + (size_t)M * sizeof(int));
     const size_t o_x = al(o_bad + (size_t)M * sizeof(int));
     const size_t o_p = al(o_x + (copy_x ? (size_t)(M * K) * sizeof(float) : 0));
@@ -646,13 +689,14 @@ int launch_fast_gemm(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_
     }
     float *pm = reinterpret_cast<float *>(ws + o_pm);
     int *ex = reinterpret_cast<int *>(ws + o_ex), *bad = reinterpret_cast<int *>(ws + o_bad);
-    hipLaunchKernelGGL(row_max_kernel, dim3((unsigned)((M * np + 3) / 4)), dim3(256), 0, ctx->stream, xa, M, K, np, pm);
-    if (w->dtype == kQ4K)
-        hipLaunchKernelGGL(split_kernel<true>, dim3((unsigned)(mt * nch)), dim3(256), 0, ctx->stream, xa, M, K, np, pm, ws,
+    auto split = [&](auto max_kernel, auto split_kernel) {
+        hipLaunchKernelGGL(max_kernel, dim3((unsigned)((M * np + 3) / 4)), dim3(256), 0, ctx->stream, xa, M, K, np, pm);
+        hipLaunchKernelGGL(split_kernel, dim3((unsigned)(mt * nch)), dim3(256), 0, ctx->stream, xa, M, K, np, pm, ws,
                            ws + o_s, ex, bad);
-    else
-        hipLaunchKernelGGL(split_kernel<false>, dim3((unsigned)(mt * nch)), dim3(256), 0, ctx->stream, xa, M, K, np, pm, ws,
-                           ws + o_s, ex, bad);
+    };
+    if (w->dtype == kQ4K) split(row_max_kernel<false>, split_kernel<kQ4K>);
+    else if (w->dtype == kQ6K) split(row_max_kernel<false>, split_kernel<kQ6K>);
+    else split(row_max_kernel<true>, split_kernel<kQ8>);  // (as for kQ4)
     if ((st = launch_check(ctx, "fast_gemm: split")) != TRHIP_OK) return st;
     float *partial = nsl > 1 ? reinterpret_cast<float *>(ws + o_p) : nullptr;
 #define TRHIP_FG(DT) st = run_dt<DT>(ctx, w, row0, N, xa, ws, ws + o_s, ex, bad, cps, nsl, c, partial, M, acc, wm)

@@ -1,7 +1,7 @@
-"""Fast mode at many rows (fastg.hip, every dtype): two f16 terms of x on the matrix cores.
+"""Fast mode at many rows (fastg.hip, every dtype): x as three bf16 terms (q8_0, q4_0) or two f16 ones on the matrix cores.
 
-Bounds. Against float64, the product of the dequantized weights: x is split to 2^-23 of each element, products are
-exact, and what rounds is fp32 sums no longer than the exact mode's chains, so the relative error (2-norm) stays below
+Bounds. Against float64, the product of the dequantized weights: x is split exactly or to 2^-23 of each element, products
+are exact, and what rounds is fp32 sums no longer than the exact mode's chains, so the relative error (2-norm) stays below
 the exact mode's own on the same inputs (measured 0.3 to 0.7 of it); the test allows equality. Per element the header's
 bound, |a - b| / (1 + |b|) <= 1e-5 (q8_0, q4_0) / 1e-4 (q4_k, q6_k) of the oracle, at x1 and x1000."""
 import numpy as np
@@ -112,3 +112,53 @@ def test_fast_gemm_swiglu(backend, dt, M, I, K):
     for b in (xb, ob):
         b.free()
     w.release()
+
+
+def _outlier_case(dt, M, N, K, big):
+    """x of order 1 with one element of `big` in every row; the weights at that element are zero, so no output depends on it."""
+    raw = synth.quant_weights(dt, N, K, seed=K + N, outliers=0.01)
+    x = synth.activations(M, K, seed=M)
+    k = K // 2 + 37
+    rows = raw.reshape(N, -1)
+    if dt == Q8:
+        rows[:, k // 32 * 34 + 2 + k % 32] = 0
+    else:
+        j = k // 32 * 18 + 2 + k % 16
+        rows[:, j] = (rows[:, j] & 0xF0 | 8) if k % 32 < 16 else (rows[:, j] & 0x0F | 0x80)
+    assert not O.dequant(dt, raw).reshape(N, K)[:, k].any()
+    x[:, k] = np.float32(big)
+    return raw, x
+
+
+@pytest.mark.parametrize("dt,M,N", [(Q8, 130, 1024), (Q4, 130, 1024)])
+@pytest.mark.parametrize("big", [1e8, -1e20, 1e30])
+def test_fast_gemm_outlier(backend, dt, M, N, big):
+    """The header's bound, |a - b| / (1 + |b|), unscaled, where one element is 1e8 to 1e30 times the others."""
+    K = 4096
+    raw, x = _outlier_case(dt, M, N, K, big)
+    w = backend.FromQuantized(dt, raw, N, K)
+    got = _call(backend, w, x, 0, N, K, np.zeros((M, N), np.float32), 0, False)
+    pick = [0, 31, 32, M - 1]
+    want = O.quant_gemm(dt, len(pick), N, K, x[pick], raw).reshape(len(pick), N)
+    assert np.abs(want).max() > 0.1
+    assert rel_err(got[pick], want) <= TOL[dt]
+    w.release()
+
+
+@pytest.mark.parametrize("dt", [Q8, Q4])
+def test_fast_gemm_nonfinite_rows(backend, dt):
+    """q8_0 / q4_0 take NaN and Inf as ordinary terms: every row non-finite in some way (NaNs whose payload is all in the low
+    16 bits too), K in slices and not. A row's outputs are NaN or infinite where the oracle's are, its sign included."""
+    for N, K in ((500, 4096), (300, 256)):
+        M = 64
+        raw = synth.quant_weights(dt, N, K, seed=5, outliers=0.01)
+        w = backend.FromQuantized(dt, raw, N, K)
+        x = synth.activations(M, K, seed=6)
+        x.view(np.uint32)[np.arange(M), np.arange(M) * 3] = [(0x7F800001, 0xFFC00000, 0x7F800000, 0xFF800000)[m % 4] for m in range(M)]
+        x[3::8, 200] = np.inf
+        x[5] = np.nan
+        got = _call(backend, w, x, 0, N, K, np.zeros((M, N), np.float32), 0, False)
+        want = O.quant_gemm(dt, M, N, K, x, raw).reshape(M, N)
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        assert not np.isfinite(want).any() and np.array_equal(got[~np.isnan(want)], want[~np.isnan(want)])
+        w.release()
