@@ -2,13 +2,15 @@
 // matrix cores: trhip_gemm_q(TRHIP_MODE_FAST). The reference's GPU runs these as dequantized tiles through a float GEMM
 // (gpu/backend_quant.go:43-134), a tolerance path too.
 //
-// Activations: each row is scaled by a power of two, x' = x 2^(14 - E) with 2^E > max|x| of the row, and split.
-//   q8_0, q4_0: three bf16 terms of eight bits, which add up to x' exactly, whatever the range of the row (bf16 has fp32's
+// Activations: x is scaled by a power of two, x' = x 2^(14 - E), and split into terms.
+//   q8_0, q4_0: 2^E > max|x| of the row; three bf16 terms of eight bits, which add up to x' exactly, whatever the range of the row (bf16 has fp32's
 //     exponents; elements below 2^-110 of the row's largest lose low bits). Two f16 terms, exact to 2^-39 of the row's
 //     largest only, were 10-25% faster (4096 x 14336, M = 300 134 against 164 us) and lost every element beside one 2^40
 //     times larger.
-//   q4_k, q6_k: two f16 terms, hi = f16(x') and lo = f16(x' - hi): exact to 2^-23 of each element, and to 2^-39 of the
-//     row's largest where lo is subnormal (the f16 MFMAs keep subnormals).
+//   q4_k, q6_k: 2^E > max|x| of the row's 256-element block, which each block is multiplied back by where it is folded (one
+//     exponent a row loses the other blocks of a row that holds an outlier: a row of order 1 with one element of 1e8 was
+//     off by 9e-4). Two f16 terms, hi = f16(x') and lo = f16(x' - hi): exact to 2^-23 of each element, and to 2^-39 of
+//     the block's largest where lo is subnormal (the f16 MFMAs keep subnormals).
 // Weights: the integer part of every format is exact in the terms' type,
 //   q8_0, q4_0: the code (q4 - 8);   q4_k: q4 sc - o;   q6_k: (q6 - 32) (sc & ~1) and (q6 - 32) (sc & 1), two planes
 // so each product is exact and only fp32 sums round. Per block (32 elements for q8_0 and q4_0, 256 for the k-quants)
@@ -101,8 +103,8 @@ __global__ __launch_bounds__(256) void row_max_kernel(const float *__restrict__ 
 template <int DT>
 __global__ __launch_bounds__(256) void split_kernel(const float *__restrict__ x, int64_t M, int64_t K, int64_t np,
                                                     const float *__restrict__ pm, uint8_t *__restrict__ rec,
-                                                    uint8_t *__restrict__ srec, int *__restrict__ ex,
-                                                    int *__restrict__ bad) {
+                                                    uint8_t *__restrict__ srec, float *__restrict__ sx,
+                                                    int *__restrict__ ex, int *__restrict__ bad) {
     constexpr bool SUMS = DT == kQ4K;
     constexpr int TERMS = Fg<DT>::TERMS;
     const int tid = threadIdx.x, r = tid >> 3, s8 = tid & 7;
@@ -121,14 +123,39 @@ __global__ __launch_bounds__(256) void split_kernel(const float *__restrict__ x,
         if (Fg<DT>::KQ) bad[m] = inf ? 1 : 0;
     }
     const bool use = row && !inf;
+    float4 in4[4][2];
+    auto load = [&](int j) {
+        const int64_t k = 256 * ch + 64 * j + 8 * s8;
+        const float4 *p = reinterpret_cast<const float4 *>(x + (use && k < K ? m * K + k : 0));
+        in4[j][0] = p[0];
+        in4[j][1] = p[1];
+    };
+    if (Fg<DT>::KQ) {  // the block's own exponent (K is a multiple of 256)
+        float b = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            load(j);
+            b = fmaxf(b, fmaxf(amax4(in4[j][0]), amax4(in4[j][1])));
+        }
+#pragma unroll
+        for (int o = 1; o < 8; o <<= 1) b = fmaxf(b, __shfl_xor(b, o));
+        int eb = E - 120;
+        if (use && b > 0.0f) {
+            int e = 0;
+            (void)frexpf(b, &e);
+            if (e > eb) eb = e;
+        }
+        if (s8 == 0) sx[(mt * nch + ch) * 32 + r] = ldexpf(1.0f, eb - E);
+        E = eb;
+    }
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const int64_t k = 256 * ch + 64 * j + 8 * s8;
         if (k - 8 * s8 >= 16 * KS) break;  // past the padded row (uniform)
         float v[8];
         const bool in = use && k < K;
-        const float4 *p = reinterpret_cast<const float4 *>(x + (in ? m * K + k : 0));
-        const float4 v0 = p[0], v1 = p[1];
+        if (!Fg<DT>::KQ) load(j);
+        const float4 v0 = in4[j][0], v1 = in4[j][1];
         const float raw[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
         uint16_t tm[TERMS][8];
         double s = 0.0;
@@ -389,8 +416,8 @@ struct ColW<kQ6K> {
 template <int DT, int WM, int CT>
 __global__ __launch_bounds__(FG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void fast_gemm(
     const Planes p, int64_t N, int64_t row0, int64_t M, int64_t K, const float *__restrict__ x,
-    const uint8_t *__restrict__ rec, const uint8_t *__restrict__ srec, const int *__restrict__ ex,
-    const int *__restrict__ bad, int64_t cps, float *__restrict__ c, float *__restrict__ partial, int acc_c) {
+    const uint8_t *__restrict__ rec, const uint8_t *__restrict__ srec, const float *__restrict__ sx,
+    const int *__restrict__ ex, const int *__restrict__ bad, int64_t cps, float *__restrict__ c, float *__restrict__ partial, int acc_c) {
     using L = Fg<DT>;
     constexpr bool KQ = L::KQ;
     constexpr int TM = 32 * WM, PL = L::PL, TERMS = L::TERMS;
@@ -452,9 +479,16 @@ __global__ __launch_bounds__(FG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
         for (int t = 0; t < TERMS; t++) A[ks][t] = *reinterpret_cast<const v8h *>(an + 1024 * t + l16);
     };
 
-    // Fold block ch (k-quants) into the sums.
+    // Fold block ch (k-quants) into the sums: its value times the power of two of (activation row, block).
     auto fold = [&](int ch) {
         const uint8_t *kb = blkp(ch & 1);
+        const float4 *xp = reinterpret_cast<const float4 *>(sx + (mt * nch + ch) * 32) + (lane >> 5);
+        float s8[16];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const float4 u = xp[2 * q];
+            s8[4 * q] = u.x, s8[4 * q + 1] = u.y, s8[4 * q + 2] = u.z, s8[4 * q + 3] = u.w;
+        }
         const float *dk = reinterpret_cast<const float *>(kb + L::CO) + 32 * CT * wn + (lane & 31);
         if constexpr (DT == kQ4K) {
             const v8h *so = reinterpret_cast<const v8h *>(srec + (mt * nch + ch) * 2048) + lane;
@@ -467,14 +501,14 @@ __global__ __launch_bounds__(FG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
                 V = __builtin_amdgcn_mfma_f32_32x32x16_f16(S0, vh, V, 0, 0, 0);
                 const float dv = dk[32 * t], sv = dk[FG_TN + 32 * t];
 #pragma unroll
-                for (int v = 0; v < 16; v++) acc[t][v] = fmaf(dv, D[t][v], fmaf(sv, V[v], acc[t][v]));
+                for (int v = 0; v < 16; v++) acc[t][v] = fmaf(fmaf(dv, D[t][v], sv * V[v]), s8[v], acc[t][v]);
             }
         } else if constexpr (DT == kQ6K) {
 #pragma unroll
             for (int t = 0; t < CT; t++) {
                 const float dv = dk[32 * t];
 #pragma unroll
-                for (int v = 0; v < 16; v++) acc[t][v] = fmaf(dv, D[t][v], acc[t][v]);
+                for (int v = 0; v < 16; v++) acc[t][v] = fmaf(dv, D[t][v] * s8[v], acc[t][v]);
             }
         }
     };
@@ -621,7 +655,7 @@ __global__ __launch_bounds__(256) void slice_sum(const float *__restrict__ parti
 
 template <int DT, int WM, int CT>
 int run(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, const uint8_t *rec,
-        const uint8_t *srec, const int *ex, const int *bad, int64_t cps, int64_t nsl, float *c, float *partial, int64_t M,
+        const uint8_t *srec, const float *sx, const int *ex, const int *bad, int64_t cps, int64_t nsl, float *c, float *partial, int64_t M,
         bool acc) {
     const auto kern = &fast_gemm<DT, WM, CT>;
     const int st = allow_dyn_lds(ctx, reinterpret_cast<const void *>(kern), Fg<DT>::LDS, "fast_gemm: LDS size");
@@ -629,17 +663,17 @@ int run(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const fl
     const int64_t tiles = ((M + 32 * WM - 1) / (32 * WM)) * ((N + FG_TN - 1) / FG_TN);
     if (tiles >= ((int64_t)1 << 31)) return fail(ctx, TRHIP_ERR_UNSUPPORTED, "fast_gemm: grid too large");
     hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)nsl), dim3(FG_THREADS), Fg<DT>::LDS, ctx->stream, w->planes(),
-                       N, row0, M, w->K, x, rec, srec, ex, bad, cps, c, partial, acc ? 1 : 0);
+                       N, row0, M, w->K, x, rec, srec, sx, ex, bad, cps, c, partial, acc ? 1 : 0);
     return launch_check(ctx, "fast_gemm");
 }
 
 template <int DT>
 int run_dt(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, const uint8_t *rec,
-           const uint8_t *srec, const int *ex, const int *bad, int64_t cps, int64_t nsl, float *c, float *partial,
+           const uint8_t *srec, const float *sx, const int *ex, const int *bad, int64_t cps, int64_t nsl, float *c, float *partial,
            int64_t M, bool acc, int wm) {
-    if (wm == 1) return run<DT, 1, 1>(ctx, w, row0, N, x, rec, srec, ex, bad, cps, nsl, c, partial, M, acc);
-    if (wm == 2) return run<DT, 2, 2>(ctx, w, row0, N, x, rec, srec, ex, bad, cps, nsl, c, partial, M, acc);
-    return run<DT, 4, 4>(ctx, w, row0, N, x, rec, srec, ex, bad, cps, nsl, c, partial, M, acc);
+    if (wm == 1) return run<DT, 1, 1>(ctx, w, row0, N, x, rec, srec, sx, ex, bad, cps, nsl, c, partial, M, acc);
+    if (wm == 2) return run<DT, 2, 2>(ctx, w, row0, N, x, rec, srec, sx, ex, bad, cps, nsl, c, partial, M, acc);
+    return run<DT, 4, 4>(ctx, w, row0, N, x, rec, srec, sx, ex, bad, cps, nsl, c, partial, M, acc);
 }
 
 }  // namespace
@@ -673,7 +707,9 @@ int launch_fast_gemm(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_
     auto al = [](size_t v) { return (v + 255) / 256 * 256; };
     const bool copy_x = reinterpret_cast<uintptr_t>(x) % 16 != 0;
     const bool kq = w->dtype == kQ4K || w->dtype == kQ6K;
-    const size_t o_s = al((size_t)(mt * KS) * (kq ? 2048 : 3072)), o_pm = al(o_s + (w->dtype == kQ4K ? (size_t)(mt * nch) * 2048 : 0));
+    const size_t o_s = al((size_t)(mt * KS) * (kq ? 2048 : 3072));
+    const size_t o_sx = al(o_s + (w->dtype == kQ4K ? (size_t)(mt * nch) * 2048 : 0));
+    const size_t o_pm = al(o_sx + (kq ? (size_t)(mt * nch) * 32 * sizeof(float) : 0));
     const size_t o_ex = al(o_pm + (size_t)(M * np) * sizeof(float)), o_bad = al(o_ex + (size_t)M * sizeof(int));
     const size_t o_x = al(o_bad + (size_t)M * sizeof(int));
     const size_t o_p = al(o_x + (copy_x ? (size_t)(M * K) * sizeof(float) : 0));
@@ -687,19 +723,19 @@ int launch_fast_gemm(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_
         if (e != hipSuccess) return hip_fail(ctx, e, "fast_gemm: align x");
         xa = reinterpret_cast<const float *>(ws + o_x);
     }
-    float *pm = reinterpret_cast<float *>(ws + o_pm);
+    float *pm = reinterpret_cast<float *>(ws + o_pm), *sx = reinterpret_cast<float *>(ws + o_sx);
     int *ex = reinterpret_cast<int *>(ws + o_ex), *bad = reinterpret_cast<int *>(ws + o_bad);
     auto split = [&](auto max_kernel, auto split_kernel) {
         hipLaunchKernelGGL(max_kernel, dim3((unsigned)((M * np + 3) / 4)), dim3(256), 0, ctx->stream, xa, M, K, np, pm);
         hipLaunchKernelGGL(split_kernel, dim3((unsigned)(mt * nch)), dim3(256), 0, ctx->stream, xa, M, K, np, pm, ws,
-                           ws + o_s, ex, bad);
+                           ws + o_s, sx, ex, bad);
     };
     if (w->dtype == kQ4K) split(row_max_kernel<false>, split_kernel<kQ4K>);
     else if (w->dtype == kQ6K) split(row_max_kernel<false>, split_kernel<kQ6K>);
     else split(row_max_kernel<true>, split_kernel<kQ8>);  // (as for kQ4)
     if ((st = launch_check(ctx, "fast_gemm: split")) != TRHIP_OK) return st;
     float *partial = nsl > 1 ? reinterpret_cast<float *>(ws + o_p) : nullptr;
-#define TRHIP_FG(DT) st = run_dt<DT>(ctx, w, row0, N, xa, ws, ws + o_s, ex, bad, cps, nsl, c, partial, M, acc, wm)
+#define TRHIP_FG(DT) st = run_dt<DT>(ctx, w, row0, N, xa, ws, ws + o_s, sx, ex, bad, cps, nsl, c, partial, M, acc, wm)
     switch (w->dtype) {
     case kQ8: TRHIP_FG(kQ8); break;
     case kQ4: TRHIP_FG(kQ4); break;

@@ -115,22 +115,27 @@ def test_fast_gemm_swiglu(backend, dt, M, I, K):
 
 
 def _outlier_case(dt, M, N, K, big):
-    """x of order 1 with one element of `big` in every row; the weights at that element are zero, so no output depends on it."""
+    """x of order 1 with one element of `big` in every row; the weights at that element are zero, so no output depends on
+    it. q4_k / q6_k, which keep 24 bits of a 256-element block's largest value: the whole block's are zero."""
     raw = synth.quant_weights(dt, N, K, seed=K + N, outliers=0.01)
     x = synth.activations(M, K, seed=M)
     k = K // 2 + 37
     rows = raw.reshape(N, -1)
     if dt == Q8:
         rows[:, k // 32 * 34 + 2 + k % 32] = 0
-    else:
+    elif dt == Q4:
         j = k // 32 * 18 + 2 + k % 16
         rows[:, j] = (rows[:, j] & 0xF0 | 8) if k % 32 < 16 else (rows[:, j] & 0x0F | 0x80)
+    elif dt == Q4K:
+        rows[:, k // 256 * 144 + 4:(k // 256 + 1) * 144] = 0  # scales, minimums and codes
+    else:
+        rows[:, k // 256 * 210:k // 256 * 210 + 192] = np.r_[np.zeros(128), np.full(64, 0xAA)].astype(np.uint8)  # codes 32
     assert not O.dequant(dt, raw).reshape(N, K)[:, k].any()
     x[:, k] = np.float32(big)
     return raw, x
 
 
-@pytest.mark.parametrize("dt,M,N", [(Q8, 130, 1024), (Q4, 130, 1024)])
+@pytest.mark.parametrize("dt,M,N", [(Q8, 130, 1024), (Q4, 130, 1024), (Q4K, 300, 6400), (Q6K, 300, 4096)])
 @pytest.mark.parametrize("big", [1e8, -1e20, 1e30])
 def test_fast_gemm_outlier(backend, dt, M, N, big):
     """The header's bound, |a - b| / (1 + |b|), unscaled, where one element is 1e8 to 1e30 times the others."""
