@@ -239,6 +239,12 @@ int trhip_mfma_probe(trhip_ctx *ctx, int valu_per_mfma, int waves_per_simd, int6
  * ceiling of the loop the prefill kernel runs per block. Refused during graph capture. */
 int trhip_prefill_probe(trhip_ctx *ctx, int kind, int64_t M, int64_t N, int64_t K);
 
+/* Diagnostic with no counterpart in the reference, on the host alone: how an exact product of M > 1 activation rows with N
+ * weight rows of K elements is cut on a device of `cus` CUs. plan[0]: K slices (1: a row block's chunks in one
+ * workgroup), plan[1]: activation rows a pass (16 or 32; of up to 16 rows, one pass), plan[2]: workgroups the passes
+ * are dealt over. Every cut gives the same bits. */
+int trhip_rows_plan(int dtype, int64_t M, int64_t N, int64_t K, int cus, int64_t *plan);
+
 /* Test and tuning hook with no counterpart in the reference: force a launch shape on this context
  * instead of the built-in choice (all four values 0 restores it). Shapes that are not built are
  * refused here, never at a later GEMV. TRHIP_KNOB_KL: K-across-lanes fast GEMV (a, b, c, d) =
@@ -247,9 +253,11 @@ int trhip_prefill_probe(trhip_ctx *ctx, int kind, int64_t M, int64_t N, int64_t 
  * per workgroup a; TRHIP_KNOB_EXACT_LANES: exact GEMV lanes per row a (4, 8 or 16); TRHIP_KNOB_ACTQ_TM: act-quant
  * MFMA row tile a (0: built-in) and, in fast mode, b K slices (0: built-in); TRHIP_KNOB_ROWS16: fast q4_k kernel for 2..16 activation rows (a, b) = (16-row tiles per
  * wave 1 or 2; K slices 1..64, clamped to the block count); TRHIP_KNOB_KL_GRID: at least a workgroups for
- * the K-across-lanes fast GEMV (its rows dealt over more, shorter row groups). */
+ * the K-across-lanes fast GEMV (its rows dealt over more, shorter row groups); TRHIP_KNOB_ROWS: exact products of more
+ * than 16 activation rows (a, b, c) = (1: a row block's K chunks in one workgroup, 2: in slices where there are
+ * enough of them; activation rows a pass, 16 or 32; workgroups its passes are dealt over). */
 enum { TRHIP_KNOB_KL = 1, TRHIP_KNOB_FAST_Q4K = 2, TRHIP_KNOB_EXACT_ROWS = 3, TRHIP_KNOB_EXACT_LANES = 4,
-       TRHIP_KNOB_ACTQ_TM = 5, TRHIP_KNOB_ROWS16 = 6, TRHIP_KNOB_KL_GRID = 7 };
+       TRHIP_KNOB_ACTQ_TM = 5, TRHIP_KNOB_ROWS16 = 6, TRHIP_KNOB_KL_GRID = 7, TRHIP_KNOB_ROWS = 8 };
 int trhip_set_launch_shape(trhip_ctx *ctx, int knob, int a, int b, int c, int d);
 
 #ifdef __cplusplus

@@ -59,6 +59,7 @@ SIGNATURES = [
     ("trhip_quantize_q8", INT, [P, P, I64, I64, INT, P, P, P]),
     ("trhip_swiglu", INT, [P, P, I64, I64, P]),
     ("trhip_gemm_q_swiglu", INT, [P, P, P, P, I64, I64, INT]),
+    ("trhip_rows_plan", INT, [INT, I64, I64, I64, INT, ctypes.POINTER(I64)]),
     ("trhip_set_launch_shape", INT, [P, INT, INT, INT, INT, INT]),
 ]
 
@@ -67,7 +68,7 @@ OK, ERR_INVALID, ERR_OOM, ERR_HIP, ERR_LAUNCH, ERR_UNSUPPORTED, ERR_NO_DEVICE, E
 Q8, Q4, Q4K, Q6K = 1, 2, 3, 4
 MODE_EXACT, MODE_FAST = 0, 1
 F32, F16, BF16 = 0, 1, 2
-KNOB_KL, KNOB_FAST_Q4K, KNOB_EXACT_ROWS, KNOB_EXACT_LANES, KNOB_ACTQ_TM, KNOB_ROWS16, KNOB_KL_GRID = 1, 2, 3, 4, 5, 6, 7
+KNOB_KL, KNOB_FAST_Q4K, KNOB_EXACT_ROWS, KNOB_EXACT_LANES, KNOB_ACTQ_TM, KNOB_ROWS16, KNOB_KL_GRID, KNOB_ROWS = range(1, 9)
 
 
 def load(path=LIB_PATH):

@@ -521,6 +521,12 @@ int trhip_graph_destroy(void *exec) {
     return e2 == hipSuccess ? TRHIP_OK : hip_fail(ctx, e2, "graph destroy");
 }
 
+int trhip_rows_plan(int dtype, int64_t M, int64_t N, int64_t K, int cus, int64_t *plan) {
+    if (bad_dtype(dtype) || M < 2 || N < 1 || K < 1 || K % block_elems(dtype) || cus < 1 || !plan) return TRHIP_ERR_INVALID;
+    gemm_rows_cut(dtype, M, N, K, cus, plan);
+    return TRHIP_OK;
+}
+
 int trhip_set_launch_shape(trhip_ctx *ctx, int knob, int a, int b, int c, int d) {
     if (!ctx) return TRHIP_ERR_INVALID;
     const bool reset = a == 0 && b == 0 && c == 0 && d == 0;
@@ -564,6 +570,13 @@ int trhip_set_launch_shape(trhip_ctx *ctx, int knob, int a, int b, int c, int d)
         if (!(reset || (a >= 1 && a <= 65536 && !b && !c && !d)))
             return fail(ctx, TRHIP_ERR_INVALID, "set_launch_shape: K-across-lanes grid takes 1..65536 workgroups");
         ctx->kl_min_wgs = a;
+        return TRHIP_OK;
+    case TRHIP_KNOB_ROWS:
+        if (!(reset || ((a == 1 || a == 2) && (b == 16 || b == 32) && c >= 1 && c <= 65535 && !d)))
+            return fail(ctx, TRHIP_ERR_INVALID, "set_launch_shape: rows plan takes 1..2, 16 or 32 rows, 1..65535 workgroups");
+        ctx->force_rows[0] = a;
+        ctx->force_rows[1] = b;
+        ctx->force_rows[2] = c;
         return TRHIP_OK;
     case TRHIP_KNOB_ROWS16:
         if (!(reset || ((a == 1 || a == 2) && b >= 1 && b <= 64 && !c && !d)))

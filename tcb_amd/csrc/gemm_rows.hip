@@ -349,6 +349,12 @@ __device__ __forceinline__ void put_c(void *c, int64_t i, float v, const RowsIo 
     }
 }
 
+// Two-tile workgroups of four waves in q4_0 and q4_k are held to two waves a SIMD (left alone they take 297 registers and
+// run one: 8192 x 8192, M = 200 488 us against 348 in seven workgroups a slice); q8_0 and q6_k would spill a hundred
+// (4096 x 4096, M = 17 q8_0 25 us against 36).
+template <int DT, int MT, int W>
+constexpr int rows_waves() { return W == kStageWaves || (MT < 0 && (DT == kQ4 || DT == kQ4K)) ? 2 : 1; }
+
 // The same chains on the matrix cores, a pass of Tiles<MT>::kRows activation rows at a time, in ascending k from +0
 // as the CPU kernel does. Activation rows past M repeat row M - 1; their results are dropped.
 //
@@ -360,9 +366,9 @@ __device__ __forceinline__ void put_c(void *c, int64_t i, float v, const RowsIo 
 // the workgroup covers every chunk and adds the chain results to `part` in chunk order in LDS; otherwise each
 // chain result goes to partial[chunk][m][row] for sum_chunks_kernel.
 template <int DT, bool X16, int MT, int W>
-__global__ __launch_bounds__(64 * W) void gemm_rows_mfma(const Planes p, const void *__restrict__ xv,
-                                                         void *__restrict__ c, float *__restrict__ partial, int64_t N,
-                                                         int64_t row0, int64_t M, int64_t K, int64_t cps, RowsIo io) {
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(rows_waves<DT, MT, W>()))) void gemm_rows_mfma(
+    const Planes p, const void *__restrict__ xv, void *__restrict__ c, float *__restrict__ partial, int64_t N, int64_t row0,
+    int64_t M, int64_t K, int64_t cps, RowsIo io) {
     using XT = std::conditional_t<X16, uint16_t, float>;
     using XP = std::conditional_t<X16, u32x2, f32x4>;  // four activations as loaded
     const XT *x = static_cast<const XT *>(xv);
@@ -558,23 +564,64 @@ int run_dt(const RowsCall &r) {
 // there are enough row blocks to occupy the device; otherwise the chunks are split into slices of kSplitWaves chunks
 // (about two workgroups per CU in all) whose chain results are added in chunk order by sum_chunks_kernel.
 //
-// More rows: the plan of least estimated time. Registers and LDS hold two waves a SIMD, i.e. one workgroup of kStageWaves
-// or two of kSplitWaves a CU; so a plan takes ceil(workgroups / slots) rounds, a round the passes and chunk turns of one
-// workgroup. What a turn takes (two waves a SIMD; us for 16 rows and for 32, whose weights are decoded once) is measured
-// per format, in the larger workgroups with their sums in LDS and in the smaller ones; partial chain results cost a
-// launch, a write and a read. Passes dealt over workgroups instead of walked by one fill the device where row blocks are
-// few: 4096 x 4096, M = 77 (q4_k) 53 us walked, 41 in two workgroups per slice; 1024 x 4096, M = 300 172 walked, 50
-// dealt; 14336 x 4096, M = 512 862 walked in 16s, 655 dealt in 32s (784 dealt in 16s).
-struct TurnCost {
-    double whole[2], split[2];  // 16 rows, 32 rows
+// More rows: the plan of least estimated time, unless the walked one (16-row passes, one workgroup a row block and slice) is
+// within 6% of it. The costs below are fitted to 18 thousand measured times (four formats, 256 to 28672 rows, 17 to 1024
+// activation rows, cold weights): the plan taken is 1.1% over the best one in the mean, 15% at most, and over the walked
+// one at 1 of 1148 sizes by more than 3%. (Turns of one workgroup of kStageWaves or two of kSplitWaves a CU for every
+// format, in whole rounds, had put it over the walked plan by up to 32% at 76 of them: 4096 x 4096, M = 77, q8_0 55 -> 73.)
+//
+// A CU holds one workgroup of kStageWaves, and of kSplitWaves as many as their registers leave: two for q4_0 and q4_k, one
+// for q8_0 and q6_k (more than 256 registers a wave). Passes dealt over workgroups instead of walked by one fill the device
+// where row blocks are few: q4_k 4096 x 4096, M = 77 53 us walked, 41 in two workgroups per slice; 1024 x 4096, M = 300 172
+// walked, 48 dealt; 14336 x 4096, M = 512 864 walked in 16s, 661 dealt in 32s.
+struct TurnCost {                        // us for a turn on 16 and on 32 activation rows (whose weights are decoded once)
+    double whole[2], alone[2], pair[2];  // a workgroup of kStageWaves; of kSplitWaves, one and two on a CU
+    double start[2], slice_start, pass;  // the start of a workgroup of kStageWaves, of kSplitWaves; of a pass
+    double later, half;                  // share of a start that shows after the first; of a tile that a half pass saves
+    double sums, l2_rate, rate;          // the partial sums' launch; MB / us of those that the L2s hold, of the rest
 };
 TurnCost turn_cost(int dtype) {
-    if (dtype == kQ8) return {{15.9, 29.5}, {17.5, 29.0}};
-    if (dtype == kQ6K) return {{18.0, 31.0}, {20.0, 33.0}};
-    return {{14.0, 24.0}, {12.5, 22.0}};
+    if (dtype == kQ8) return {{14.2, 25.1}, {7.7, 12.6}, {0, 0}, {6.8, 14.7}, 1.0, 1.2, 0.58, 0.7, 7.46, 4.6, 2.4};
+    if (dtype == kQ6K) return {{16.2, 29.0}, {9.1, 14.2}, {0, 0}, {6.0, 12.4}, 0.9, 0.9, 0.52, 0.58, 7.9, 4.0, 2.9};
+    return {{10.8, 18.4}, {5.9, 11.0}, {8.7, 16.2}, {3.9, 5.3}, 0.9, 0.9, 0.42, 0.68, 6.8, 5.8, 2.3};
+}
+constexpr bool two_split_workgroups(int dtype) { return dtype == kQ4 || dtype == kQ4K; }
+
+// Passes one after another until the last of B workgroups for each of z ends, `slots` at a time in grid order: the first
+// np % z of the z take a pass more.
+int64_t passes_in_turn(int64_t B, int64_t np, int64_t z, int64_t slots) {
+    const int64_t q = np / z, heavy = np % z * B, f = heavy / slots, l = heavy % slots, rest = z * B - f * slots;
+    const int64_t t = f * (q + 1);
+    if (rest <= 0) return t;
+    const int64_t n = (rest + slots - 1) / slots, last = rest - (n - 1) * slots;
+    if (l == 0) return t + n * q;
+    if (n == 1) return t + q + 1;
+    if (last > slots - l) return t + q + 1 + (n - 1) * q;
+    return t + (n * q > q + 1 + (n - 2) * q ? n * q : q + 1 + (n - 2) * q);
 }
 
-RowsPlan rows_plan(int dtype, int64_t M, int64_t N, int64_t nchunks, int64_t cus) {
+double plan_time(const RowsPlan &p, const TurnCost &cost, int dtype, int64_t M, int64_t N, int64_t nchunks, int64_t cus) {
+    const bool cut = p.nslices > 1;
+    const int64_t nrb = (N + 63) / 64, B = nrb * p.nslices, waves = cut ? kSplitWaves : kStageWaves;
+    const int64_t np = (M + (p.two ? 31 : 15)) / (p.two ? 32 : 16), turns = (p.cps + waves - 1) / waves;
+    const bool pair = cut && two_split_workgroups(dtype) && B * p.pz > cus;
+    // (up to kSplitWaves chunks leave a workgroup of kStageWaves one wave a SIMD)
+    const double *turn = pair ? cost.pair : cut || nchunks <= kSplitWaves ? cost.alone : cost.whole;
+    const int64_t slots = pair ? 2 * cus : cus, rounds = (B * p.pz + slots - 1) / slots;
+    double t = (double)passes_in_turn(B, np, p.pz, slots) * ((double)turns * turn[p.two] + cost.pass);
+    // (a start after the first overlaps the other workgroups' work in part)
+    t += (1.0 + cost.later * (double)(rounds - 1)) * (cut ? cost.slice_start : cost.start[p.two]);
+    // half a last pass: in every round where passes are walked, in its share of the rounds where each has its workgroup
+    const double halves = p.pz == 1 ? (double)rounds : p.pz == np ? (double)B / (double)slots : 0.0;
+    if (p.two && M - 32 * (np - 1) <= 16) t -= cost.half * halves * (double)turns * (turn[1] - turn[0]);
+    if (cut) {
+        const double mb = (double)(nchunks * M * N) * 4e-6, l2 = mb < 32.0 ? mb : 32.0;
+        t += cost.sums + l2 / cost.l2_rate + (mb - l2) / cost.rate;
+    }
+    return t;
+}
+
+RowsPlan rows_plan(int dtype, int64_t M, int64_t N, int64_t nchunks, int64_t cus, const int *force = nullptr) {
     const int64_t nrb = (N + 63) / 64;
     RowsPlan split = {1, nchunks, 1, false};
     if (nchunks > kSplitWaves) {
@@ -584,29 +631,33 @@ RowsPlan rows_plan(int dtype, int64_t M, int64_t N, int64_t nchunks, int64_t cus
         split.cps = (cps + kSplitWaves - 1) / kSplitWaves * kSplitWaves;
         split.nslices = (nchunks + split.cps - 1) / split.cps;
     }
-    const RowsPlan whole = {1, nchunks, 1, false};
-    if (M <= 16) return nrb < 160 ? split : whole;
+    const RowsPlan whole = {1, nchunks, 1, false}, walked = nrb < 160 ? split : whole;
+    if (M <= 16) return walked;
+    if (force && force[0]) {
+        RowsPlan p = force[0] == 2 ? split : whole;
+        p.two = force[1] == 32;
+        const int64_t np = (M + force[1] - 1) / force[1];
+        p.pz = force[2] < np ? force[2] : np;
+        return p;
+    }
     const TurnCost cost = turn_cost(dtype);
-    RowsPlan best = whole;
-    double least = 1e30;
+    RowsPlan best = walked;
+    double least = 0.94 * plan_time(walked, cost, dtype, M, N, nchunks, cus);
     for (int cut = 0; cut < (split.nslices > 1 ? 2 : 1); cut++)
         for (int two = 0; two < 2; two++) {
             RowsPlan p = cut ? split : whole;
             p.two = two != 0;
-            const int64_t np = (M + (two ? 31 : 15)) / (two ? 32 : 16), waves = cut ? kSplitWaves : kStageWaves;
-            const int64_t slots = cus * (2 * 4 / waves), turns = (p.cps + waves - 1) / waves;
-            const double sums = cut ? 3.0 + (double)(nchunks * M * N) * 8.0 / 8e6 : 0.0;  // us, mostly cached
-            for (int64_t z = 1; z <= np && z <= 65535; z = z < 16 || z == np ? z + 1 : np) {
-                const int64_t wgs = nrb * p.nslices * z, rounds = (wgs + slots - 1) / slots, passes = (np + z - 1) / z;
-                const double alone = wgs * waves <= 4 * cus ? 0.82 : 1.0;  // one wave a SIMD
-                const double turn = alone * (cut ? cost.split[two] : cost.whole[two]);
-                // (a round's own start: its first weights and activations come from memory)
-                const double t = (double)rounds * ((double)(passes * turns) * turn + 4.0) + sums;
+            const int64_t np = (M + (two ? 31 : 15)) / (two ? 32 : 16);
+            for (int64_t z = 1; z <= 65535;) {  // the fewest workgroups for each number of passes one may take
+                p.pz = z;
+                const double t = plan_time(p, cost, dtype, M, N, nchunks, cus);
                 if (t < least) {
                     least = t;
-                    p.pz = z;
                     best = p;
                 }
+                const int64_t most = (np + z - 1) / z;
+                if (most == 1) break;
+                z = (np + most - 2) / (most - 1);
             }
         }
     return best;
@@ -614,11 +665,18 @@ RowsPlan rows_plan(int dtype, int64_t M, int64_t N, int64_t nchunks, int64_t cus
 
 }  // namespace
 
+void gemm_rows_cut(int dtype, int64_t M, int64_t N, int64_t K, int64_t cus, int64_t plan[3]) {
+    const RowsPlan p = rows_plan(dtype, M, N, (K + 255) / 256, cus);
+    plan[0] = p.nslices;
+    plan[1] = p.two ? 32 : 16;
+    plan[2] = p.pz;
+}
+
 int launch_gemm_rows(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const void *x, void *c, int64_t M,
                      bool acc, int xio, int cio) {
     if (N == 0 || M == 0) return TRHIP_OK;
     const int64_t K = w->K, nchunks = (K + 255) / 256;
-    const RowsPlan pl = rows_plan(w->dtype, M, N, nchunks, ctx->sm_count > 0 ? ctx->sm_count : 256);
+    const RowsPlan pl = rows_plan(w->dtype, M, N, nchunks, ctx->sm_count > 0 ? ctx->sm_count : 256, ctx->force_rows);
     // the kernel reads x four elements at a time
     const size_t xel = xio == TRHIP_F32 ? sizeof(float) : sizeof(uint16_t);
     const bool copy_x = reinterpret_cast<uintptr_t>(x) % (4 * xel) != 0;

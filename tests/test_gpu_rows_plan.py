@@ -1,12 +1,13 @@
 """Exact products of more than 16 activation rows: passes of 16 or 32 rows, walked by one workgroup or dealt over
-several, chunks whole or in slices. Bit-identical to the oracle whichever plan the sizes take (bit equality, so there is
-no tolerance to choose)."""
+several, chunks whole or in slices. Bit-identical to the oracle with the plan the sizes take and with each kind of plan
+forced (bit equality, so there is no tolerance to choose)."""
 import numpy as np
 import pytest
 
 import oracle as O
 from conftest import same_bits
 from tcb_amd import BF16, F16, F32, MODE_EXACT, Q4, Q4K, Q6K, Q8, synth
+from tcb_amd._lib import KNOB_ROWS
 
 pytestmark = pytest.mark.gpu
 
@@ -66,5 +67,33 @@ def test_rows_typed_bits(backend, xt, ct, dt, M, N, K, off):
         got, want = O.widen16(ct, got), O.widen16(ct, O.round16(ct, want))
     same_bits(got, want)
     for b in (xb, cb, x32, c32):
+        b.free()
+    w.release()
+
+
+# chunks whole (one or two turns of a workgroup's eight waves, the second short) or in slices (several turns of four);
+# passes of 16 and 32 rows, all walked by one workgroup, dealt one each, and several each
+PLANS = [(1, 16, 1), (1, 16, 3), (1, 32, 1), (1, 32, 2), (1, 32, 99), (2, 16, 1), (2, 16, 2), (2, 32, 1), (2, 32, 2), (2, 32, 99)]
+
+
+@pytest.mark.parametrize("dt", [Q8, Q4, Q4K, Q6K])
+@pytest.mark.parametrize("plan", PLANS)
+@pytest.mark.parametrize("M,N,K", [(97, 130, 2304), (49, 70, 4352), (41, 64, 1280)])  # last 32-row pass of 1, 17, 9 rows
+def test_forced_plan_bits(backend, launch_shape, dt, plan, M, N, K):
+    if dt in (Q8, Q4):
+        K += 96  # a short last chunk
+    raw = synth.quant_weights(dt, N, K, seed=N + K + M, outliers=0.01)
+    w = backend.FromQuantized(dt, raw, N, K)
+    x, c0 = synth.activations(M, K, seed=K + M), synth.activations(M, N, seed=N + 5).reshape(-1)
+    want = O.quant_gemm(dt, M, N, K, x, raw, c0)
+    h, hc = O.round16(BF16, x.reshape(-1)), O.round16(BF16, c0)
+    want16 = O.round16(BF16, O.quant_gemm(dt, M, N, K, O.widen16(BF16, h).reshape(M, K), raw, O.widen16(BF16, hc)))
+    xb, cb, hb, hcb = (backend.ctx.to_device(v) for v in (x, c0, h, hc))
+    launch_shape(KNOB_ROWS, *plan)
+    backend.Gemm(M, N, K, xb, w, cb)
+    same_bits(cb.download(np.float32, M * N), want)
+    backend.GemmTyped(M, N, K, hb, BF16, w, hcb, BF16, accumulate=True, mode=MODE_EXACT)
+    same_bits(O.widen16(BF16, hcb.download(np.uint16, M * N)), O.widen16(BF16, want16))
+    for b in (xb, cb, hb, hcb):
         b.free()
     w.release()
