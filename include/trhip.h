@@ -242,7 +242,8 @@ int trhip_prefill_probe(trhip_ctx *ctx, int kind, int64_t M, int64_t N, int64_t 
 /* Diagnostic with no counterpart in the reference, on the host alone: how an exact product of M > 1 activation rows with N
  * weight rows of K elements is cut on a device of `cus` CUs. plan[0]: K slices (1: a row block's chunks in one
  * workgroup), plan[1]: activation rows a pass (16 or 32; of up to 16 rows, one pass), plan[2]: workgroups the passes
- * are dealt over. Every cut gives the same bits. */
+ * are dealt over (every cut gives the same bits). plan[3]: 1 if the same call in fast mode runs on the f16 / bf16
+ * matrix-core kernel of many rows. */
 int trhip_rows_plan(int dtype, int64_t M, int64_t N, int64_t K, int cus, int64_t *plan);
 
 /* Test and tuning hook with no counterpart in the reference: force a launch shape on this context
@@ -255,9 +256,10 @@ int trhip_rows_plan(int dtype, int64_t M, int64_t N, int64_t K, int cus, int64_t
  * wave 1 or 2; K slices 1..64, clamped to the block count); TRHIP_KNOB_KL_GRID: at least a workgroups for
  * the K-across-lanes fast GEMV (its rows dealt over more, shorter row groups); TRHIP_KNOB_ROWS: exact products of more
  * than 16 activation rows (a, b, c) = (1: a row block's K chunks in one workgroup, 2: in slices where there are
- * enough of them; activation rows a pass, 16 or 32; workgroups its passes are dealt over). */
+ * enough of them; activation rows a pass, 16 or 32; workgroups its passes are dealt over); TRHIP_KNOB_FAST_GEMM: fast
+ * mode of more than 16 rows, a = 1: always the f16 / bf16 matrix-core kernel (K of 256 up), 2: never. */
 enum { TRHIP_KNOB_KL = 1, TRHIP_KNOB_FAST_Q4K = 2, TRHIP_KNOB_EXACT_ROWS = 3, TRHIP_KNOB_EXACT_LANES = 4,
-       TRHIP_KNOB_ACTQ_TM = 5, TRHIP_KNOB_ROWS16 = 6, TRHIP_KNOB_KL_GRID = 7, TRHIP_KNOB_ROWS = 8 };
+       TRHIP_KNOB_ACTQ_TM = 5, TRHIP_KNOB_ROWS16 = 6, TRHIP_KNOB_KL_GRID = 7, TRHIP_KNOB_ROWS = 8, TRHIP_KNOB_FAST_GEMM = 9 };
 int trhip_set_launch_shape(trhip_ctx *ctx, int knob, int a, int b, int c, int d);
 
 #ifdef __cplusplus

@@ -68,7 +68,7 @@ OK, ERR_INVALID, ERR_OOM, ERR_HIP, ERR_LAUNCH, ERR_UNSUPPORTED, ERR_NO_DEVICE, E
 Q8, Q4, Q4K, Q6K = 1, 2, 3, 4
 MODE_EXACT, MODE_FAST = 0, 1
 F32, F16, BF16 = 0, 1, 2
-KNOB_KL, KNOB_FAST_Q4K, KNOB_EXACT_ROWS, KNOB_EXACT_LANES, KNOB_ACTQ_TM, KNOB_ROWS16, KNOB_KL_GRID, KNOB_ROWS = range(1, 9)
+KNOB_KL, KNOB_FAST_Q4K, KNOB_EXACT_ROWS, KNOB_EXACT_LANES, KNOB_ACTQ_TM, KNOB_ROWS16, KNOB_KL_GRID, KNOB_ROWS, KNOB_FAST_GEMM = range(1, 10)
 
 
 def load(path=LIB_PATH):

@@ -524,6 +524,7 @@ int trhip_graph_destroy(void *exec) {
 int trhip_rows_plan(int dtype, int64_t M, int64_t N, int64_t K, int cus, int64_t *plan) {
     if (bad_dtype(dtype) || M < 2 || N < 1 || K < 1 || K % block_elems(dtype) || cus < 1 || !plan) return TRHIP_ERR_INVALID;
     gemm_rows_cut(dtype, M, N, K, cus, plan);
+    plan[3] = fast_gemm_pays(dtype, M, N, K, cus) ? 1 : 0;
     return TRHIP_OK;
 }
 
@@ -577,6 +578,11 @@ int trhip_set_launch_shape(trhip_ctx *ctx, int knob, int a, int b, int c, int d)
         ctx->force_rows[0] = a;
         ctx->force_rows[1] = b;
         ctx->force_rows[2] = c;
+        return TRHIP_OK;
+    case TRHIP_KNOB_FAST_GEMM:
+        if (!(reset || ((a == 1 || a == 2) && !b && !c && !d)))
+            return fail(ctx, TRHIP_ERR_INVALID, "set_launch_shape: fast kernel of many rows takes 1 (always) or 2 (never)");
+        ctx->force_fast_gemm = a;
         return TRHIP_OK;
     case TRHIP_KNOB_ROWS16:
         if (!(reset || ((a == 1 || a == 2) && b >= 1 && b <= 64 && !c && !d)))
@@ -917,7 +923,7 @@ int trhip_gemm_q(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N,
         const int r = launch_rows16(ctx, w, row0, N, x, c, M, accumulate != 0);
         if (r != -1) return r;
     }
-    if (mode == TRHIP_MODE_FAST && fast_gemm_applies(w->dtype, M, N, K))
+    if (mode == TRHIP_MODE_FAST && fast_gemm_applies(ctx, w->dtype, M, N, K))
         return launch_fast_gemm(ctx, w, row0, N, x, c, M, accumulate != 0);
     if (mode == TRHIP_MODE_FAST && ((w->dtype == TRHIP_Q4K && M > 4) || (w->dtype == TRHIP_Q6K && M > 1)))
         return launch_gemm_rows_fast(ctx, w, row0, N, x, c, M, accumulate != 0);
@@ -1021,7 +1027,7 @@ int trhip_gemm_q_swiglu(trhip_ctx *ctx, const trhip_wstore *w, const float *x, f
         const int r = launch_rows16(ctx, w, 0, w->N, x, nullptr, M, false, out);
         if (r != -1) return r;
     }
-    if (mode == TRHIP_MODE_FAST && K > 0 && fast_gemm_applies(w->dtype, M, w->N, K))
+    if (mode == TRHIP_MODE_FAST && K > 0 && fast_gemm_applies(ctx, w->dtype, M, w->N, K))
         return launch_fast_gemm(ctx, w, 0, w->N, x, gu, M, false, out);
     if (mode == TRHIP_MODE_FAST && K > 0 && ((w->dtype == TRHIP_Q4K && M > 4) || (w->dtype == TRHIP_Q6K && M > 1)))
         return launch_gemm_rows_fast(ctx, w, 0, w->N, x, gu, M, false, out);

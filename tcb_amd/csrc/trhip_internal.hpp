@@ -365,6 +365,7 @@ struct trhip_ctx {
     int force_actq_slices = 0;  // act-quant MFMA K slices, fast mode (0: built-in)
     int force_rows16 = 0;       // batched-decode q4_k kernel: 100 tiles per wave + K slices
     int force_rows[3] = {};     // exact M > 16 plan: 1 whole / 2 in slices, activation rows a pass, workgroups (0: built-in)
+    int force_fast_gemm = 0;    // fast mode of more than 16 rows: 1 fastg.hip, 2 the other kernels (0: built-in)
     // Arrival counters of kernels whose K slices are summed by the workgroup that finishes a row tile last
     // (rows16.hip): kArrivalSlots zeroed words, each returned to zero by that workgroup.
     static constexpr int64_t kArrivalSlots = 65536;
@@ -416,6 +417,8 @@ int launch_gemv_fast_swiglu(trhip_ctx *ctx, const trhip_wstore *w, const float *
 int launch_gemm_rows(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const void *x, void *c, int64_t M,
                      bool acc, int xio = TRHIP_F32, int cio = TRHIP_F32);
 // how it cuts a call: K slices, activation rows a pass, workgroups the passes are dealt over
+// estimated time of an exact call of M > 16 rows, us
+double gemm_rows_time(int dtype, int64_t M, int64_t N, int64_t K, int64_t cus);
 void gemm_rows_cut(int dtype, int64_t M, int64_t N, int64_t K, int64_t cus, int64_t plan[3]);
 // swi != nullptr (set, not accumulate; N = 2I rows [gate | up]): out swi[m, i] = silu(c[m, i]) * c[m, I + i], fused
 // into the slice sum when K is split (c is then not written), else after it
@@ -423,7 +426,8 @@ int launch_gemm_rows_fast(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, i
                           int64_t M, bool acc, float *swi = nullptr);
 // Fast mode for many rows, every dtype, on f16 matrix cores (fastg.hip): whether it takes the shape; swi as for
 // launch_gemm_rows_fast.
-bool fast_gemm_applies(int dtype, int64_t M, int64_t N, int64_t K);
+bool fast_gemm_pays(int dtype, int64_t M, int64_t N, int64_t K, int64_t cus);
+bool fast_gemm_applies(const trhip_ctx *ctx, int dtype, int64_t M, int64_t N, int64_t K);
 int launch_fast_gemm(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c, int64_t M,
                      bool acc, float *swi = nullptr);
 int launch_quantize_q8(trhip_ctx *ctx, const float *x, int64_t M, int64_t K, int blk, int8_t *q, float *d,
