@@ -923,8 +923,10 @@ int trhip_gemm_q(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N,
         const int r = launch_rows16(ctx, w, row0, N, x, c, M, accumulate != 0);
         if (r != -1) return r;
     }
-    if (mode == TRHIP_MODE_FAST && fast_gemm_applies(ctx, w->dtype, M, N, K))
-        return launch_fast_gemm(ctx, w, row0, N, x, c, M, accumulate != 0);
+    if (mode == TRHIP_MODE_FAST && fast_gemm_applies(ctx, w->dtype, M, N, K)) {
+        const int r = launch_fast_gemm(ctx, w, row0, N, x, c, M, accumulate != 0);
+        if (r != -1) return r;
+    }
     if (mode == TRHIP_MODE_FAST && ((w->dtype == TRHIP_Q4K && M > 4) || (w->dtype == TRHIP_Q6K && M > 1)))
         return launch_gemm_rows_fast(ctx, w, row0, N, x, c, M, accumulate != 0);
     return launch_gemm_rows(ctx, w, row0, N, x, c, M, accumulate != 0);
@@ -1027,8 +1029,10 @@ int trhip_gemm_q_swiglu(trhip_ctx *ctx, const trhip_wstore *w, const float *x, f
         const int r = launch_rows16(ctx, w, 0, w->N, x, nullptr, M, false, out);
         if (r != -1) return r;
     }
-    if (mode == TRHIP_MODE_FAST && K > 0 && fast_gemm_applies(ctx, w->dtype, M, w->N, K))
-        return launch_fast_gemm(ctx, w, 0, w->N, x, gu, M, false, out);
+    if (mode == TRHIP_MODE_FAST && K > 0 && fast_gemm_applies(ctx, w->dtype, M, w->N, K)) {
+        const int r = launch_fast_gemm(ctx, w, 0, w->N, x, gu, M, false, out);
+        if (r != -1) return r;
+    }
     if (mode == TRHIP_MODE_FAST && K > 0 && ((w->dtype == TRHIP_Q4K && M > 4) || (w->dtype == TRHIP_Q6K && M > 1)))
         return launch_gemm_rows_fast(ctx, w, 0, w->N, x, gu, M, false, out);
     if ((st = trhip_gemm_q(ctx, w, 0, w->N, x, gu, M, K, 0, mode)) != TRHIP_OK) return st;

@@ -758,6 +758,7 @@ int launch_fast_gemm(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_
     const size_t o_x = al(o_bad + (size_t)M * sizeof(int));
     const size_t o_p = al(o_x + (copy_x ? (size_t)(M * K) * sizeof(float) : 0));
     const size_t total = o_p + (nsl > 1 ? (size_t)(nsl * M * N) * sizeof(float) : 0);
+    if (total > ctx->ws_bytes && capturing(ctx)) return -1;
     int st = TRHIP_OK;
     uint8_t *ws = static_cast<uint8_t *>(workspace(ctx, total, &st));
     if (!ws) return st;

@@ -621,10 +621,12 @@ double plan_time(const RowsPlan &p, const TurnCost &cost, int dtype, int64_t M, 
     return t;
 }
 
-RowsPlan rows_plan(int dtype, int64_t M, int64_t N, int64_t nchunks, int64_t cus, const int *force = nullptr) {
+// uncut: only plans without partial sums
+RowsPlan rows_plan(int dtype, int64_t M, int64_t N, int64_t nchunks, int64_t cus, const int *force = nullptr,
+                   bool uncut = false) {
     const int64_t nrb = (N + 63) / 64;
     RowsPlan split = {1, nchunks, 1, false};
-    if (nchunks > kSplitWaves) {
+    if (nchunks > kSplitWaves && !uncut) {
         const int64_t want = (512 + nrb - 1) / nrb;  // slices per row block for about 512 workgroups
         const int64_t maxs = (nchunks + kSplitWaves - 1) / kSplitWaves;
         const int64_t ns = want < maxs ? want : maxs, cps = (nchunks + ns - 1) / ns;
@@ -683,11 +685,16 @@ int launch_gemm_rows(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_
                      bool acc, int xio, int cio) {
     if (N == 0 || M == 0) return TRHIP_OK;
     const int64_t K = w->K, nchunks = (K + 255) / 256;
-    const RowsPlan pl = rows_plan(w->dtype, M, N, nchunks, ctx->sm_count > 0 ? ctx->sm_count : 256, ctx->force_rows);
+    const int64_t cus = ctx->sm_count > 0 ? ctx->sm_count : 256;
+    RowsPlan pl = rows_plan(w->dtype, M, N, nchunks, cus, ctx->force_rows);
     // the kernel reads x four elements at a time
     const size_t xel = xio == TRHIP_F32 ? sizeof(float) : sizeof(uint16_t);
     const bool copy_x = reinterpret_cast<uintptr_t>(x) % (4 * xel) != 0;
     const size_t xbytes = copy_x ? ((size_t)(M * K) * xel + 255) / 256 * 256 : 0;
+    // A captured call cannot grow the workspace. From 160 row blocks the chunks need no slices, so that such a call needs
+    // none for them either.
+    if (pl.nslices > 1 && N > 159 * 64 && xbytes + (size_t)(nchunks * M * N) * sizeof(float) > ctx->ws_bytes && capturing(ctx))
+        pl = rows_plan(w->dtype, M, N, nchunks, cus, ctx->force_rows, true);
     const size_t pbytes = pl.nslices > 1 ? (size_t)(nchunks * M * N) * sizeof(float) : 0;
     int st = TRHIP_OK;
     uint8_t *ws = nullptr;

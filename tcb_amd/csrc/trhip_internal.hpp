@@ -425,7 +425,8 @@ void gemm_rows_cut(int dtype, int64_t M, int64_t N, int64_t K, int64_t cus, int6
 int launch_gemm_rows_fast(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c,
                           int64_t M, bool acc, float *swi = nullptr);
 // Fast mode for many rows, every dtype, on f16 matrix cores (fastg.hip): whether it takes the shape; swi as for
-// launch_gemm_rows_fast.
+// launch_gemm_rows_fast. A captured call whose workspace would have to grow returns -1 with nothing launched: the routes
+// below this one may need less.
 bool fast_gemm_pays(int dtype, int64_t M, int64_t N, int64_t K, int64_t cus);
 bool fast_gemm_applies(const trhip_ctx *ctx, int dtype, int64_t M, int64_t N, int64_t K);
 int launch_fast_gemm(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c, int64_t M,

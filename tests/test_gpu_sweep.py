@@ -15,7 +15,8 @@ import pytest
 
 import oracle as O
 from conftest import rel_err, same_bits
-from tcb_amd import BLOCK, MODE_EXACT, MODE_FAST, Q4K, Q6K, QuantBackend, QuantWeight, _lib, synth
+from tcb_amd import BLOCK, MODE_EXACT, MODE_FAST, Q4, Q4K, Q6K, Q8, QuantBackend, QuantWeight, _lib, synth
+from tcb_amd._lib import KNOB_FAST_GEMM, KNOB_ROWS
 
 pytestmark = pytest.mark.gpu
 
@@ -279,4 +280,39 @@ def test_graph_replay_after_workspace_growth():
         gu.release()
     finally:
         other.close()
+        tb.close()
+
+
+@pytest.mark.parametrize("dt,mode,knob", [(Q8, MODE_FAST, (KNOB_FAST_GEMM, 1)), (Q4, MODE_FAST, (KNOB_FAST_GEMM, 1)),
+                                          (Q8, MODE_EXACT, (KNOB_ROWS, 2, 32, 1)), (Q6K, MODE_EXACT, (KNOB_ROWS, 2, 16, 2))])
+def test_capture_without_eager_call(dt, mode, knob):
+    """Calls of more than 16 rows on stores of 160 row blocks and more, captured on a context that has made none before: they
+    run without a workspace where it is too small (the plans and the fast kernel that want one are forced on), and
+    every replay gives the exact mode's bits."""
+    M, N, K = 40, 10300, 2560
+    tb = QuantBackend(0)
+    try:
+        L = _lib.lib()
+        raw = synth.quant_weights(dt, N, K, seed=4, outliers=0.01)
+        w = tb.FromQuantized(dt, raw, N, K)
+        x = synth.activations(M, K, seed=5)
+        xb, cb = tb.ctx.to_device(x), tb.ctx.alloc(M * N * 4)
+        tb.ctx.set_launch_shape(*knob)
+        g = ctypes.c_void_p()
+        assert L.trhip_graph_begin(tb.ctx.h) == 0
+        try:
+            tb.GemmSet(M, N, K, xb, w, cb, mode=mode)
+        finally:
+            assert L.trhip_graph_end(tb.ctx.h, ctypes.byref(g)) == 0
+        rows = [0, 15, 16, 31, 32, M - 1]
+        want = O.quant_gemm(dt, len(rows), N, K, x[rows], raw)
+        for _ in range(3):
+            cb.fill(0xFF)
+            assert L.trhip_graph_launch(tb.ctx.h, g) == 0
+            same_bits(cb.download(np.float32, M * N).reshape(M, N)[rows], want)
+        assert L.trhip_graph_destroy(g) == 0
+        for b in (xb, cb):
+            b.free()
+        w.release()
+    finally:
         tb.close()
