@@ -1067,7 +1067,7 @@ ActqRoute actq_route(const trhip_ctx *ctx, int dtype, int64_t M, int64_t N, int6
 
 // Scratch layout of the act-quant operator: q [M][K] int8, d [M][K/blk] fp32, bs [M][K/16] int16, one NaN/Inf flag
 // byte per activation block, for q4_k the f16 msum operands [M][K/256][16], and an aligned copy of x when x is not
-// 16-byte aligned. On the tiled routes q, d and the q4_k msum operands are in the tiled layout over rows padded to whole
+// 16-byte aligned, or c lies over an x that the product kernel itself quantizes (its workgroups read x while others write c). On the tiled routes q, d and the q4_k msum operands are in the tiled layout over rows padded to whole
 // tiles (32 rows) or prefill tiles (128), and there are no 16-sums; the kernel that quantizes x itself needs none of these.
 struct ActqLayout {
     size_t o_q = 0, o_d = 0, o_bs = 0, o_fl = 0, o_sj = 0, o_x = 0, total = 0;
@@ -1075,20 +1075,26 @@ struct ActqLayout {
     ActqRoute route = ActqRoute::rows;
 };
 
-ActqLayout actq_layout(ActqRoute route, int dtype, int64_t M, int64_t K, const float *x) {
+bool lies_over(const float *c, int64_t M, int64_t N, const float *x, int64_t K) {
+    const uintptr_t xa = reinterpret_cast<uintptr_t>(x), ca = reinterpret_cast<uintptr_t>(c);
+    return xa + 4 * (uintptr_t)(M * K) > ca && ca + 4 * (uintptr_t)(M * N) > xa;
+}
+
+ActqLayout actq_layout(ActqRoute route, int dtype, int64_t M, int64_t N, int64_t K, const float *x, const float *c) {
     ActqLayout l;
     l.route = route;
     const int64_t nb = K / block_elems(dtype);
     const bool tiled = route != ActqRoute::rows;
     const int64_t pad = route == ActqRoute::tiles ? kPrefillRowPad : tiled ? 32 : 1, Mq = (M + pad - 1) / pad * pad;
-    if (route != ActqRoute::blocks || !actq_blocks_quantizes(M)) {
+    const bool in_kernel = route == ActqRoute::blocks && actq_blocks_quantizes(M);
+    if (!in_kernel) {
         l.o_d = align_up(l.o_q + (size_t)(Mq * K), 256);
         l.o_bs = align_up(l.o_d + (size_t)(Mq * nb) * sizeof(float), 256);
         l.o_fl = align_up(l.o_bs + (tiled ? 0 : (size_t)(M * (K / 16)) * sizeof(int16_t)), 256);
         l.o_sj = align_up(l.o_fl + (size_t)(M * nb), 256);
         l.o_x = align_up(l.o_sj + (dtype == TRHIP_Q4K ? (size_t)(Mq * nb) * 32 : 0), 256);
     }
-    l.copy_x = reinterpret_cast<uintptr_t>(x) % 16 != 0;
+    l.copy_x = reinterpret_cast<uintptr_t>(x) % 16 != 0 || (in_kernel && lies_over(c, M, N, x, K));
     l.total = l.o_x + (l.copy_x ? (size_t)(M * K) * sizeof(float) : 0);
     return l;
 }
@@ -1141,17 +1147,17 @@ int actq_run(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, con
 // group would write activations that later ones read, so the row-major kernels, which read x first, take the call.
 int actq_run_within(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c, int64_t M,
                     int64_t K, int accumulate, uint8_t *ws, size_t limit, bool fast) {
-    const uintptr_t xa = reinterpret_cast<uintptr_t>(x), ca = reinterpret_cast<uintptr_t>(c);
-    if (xa + 4 * (uintptr_t)(M * K) > ca && ca + 4 * (uintptr_t)(M * N) > xa)
-        return actq_run(ctx, w, row0, N, x, c, M, K, accumulate, ws, actq_layout(ActqRoute::rows, w->dtype, M, K, x), fast);
+    if (lies_over(c, M, N, x, K))
+        return actq_run(ctx, w, row0, N, x, c, M, K, accumulate, ws, actq_layout(ActqRoute::rows, w->dtype, M, N, K, x, c), fast);
     int64_t g = (M - 1) / 32 * 32;
-    while (g > 0 && actq_layout(ActqRoute::blocks, w->dtype, g, K, x).total > limit) g -= 32;
+    while (g > 0 && actq_layout(ActqRoute::blocks, w->dtype, g, N, K, x, c).total > limit) g -= 32;
     if (g == 0) g = 1;
     for (int64_t m0 = 0; m0 < M; m0 += g) {
         const int64_t m = M - m0 < g ? M - m0 : g;
         const float *xg = x + m0 * K;
-        const int st = actq_run(ctx, w, row0, N, xg, c + m0 * N, m, K, accumulate, ws,
-                                actq_layout(ActqRoute::blocks, w->dtype, m, K, xg), fast);
+        float *cg = c + m0 * N;
+        const int st = actq_run(ctx, w, row0, N, xg, cg, m, K, accumulate, ws,
+                                actq_layout(ActqRoute::blocks, w->dtype, m, N, K, xg, cg), fast);
         if (st != TRHIP_OK) return st;
     }
     return TRHIP_OK;
@@ -1194,11 +1200,11 @@ int trhip_gemm_q_actq_mode(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, 
     if (r) return st;
     DevGuard g(ctx);
     if (K == 0) return accumulate ? TRHIP_OK : zero_f32(ctx, c, M * N);
-    const ActqLayout l = actq_layout(actq_route(ctx, w->dtype, M, N, row0, K), w->dtype, M, K, x);
+    const ActqLayout l = actq_layout(actq_route(ctx, w->dtype, M, N, row0, K), w->dtype, M, N, K, x, c);
     const bool fast = mode == TRHIP_MODE_FAST;
     // a captured call cannot grow the workspace; one that holds the row-major layout is enough
     if (l.route == ActqRoute::blocks && l.total > ctx->ws_bytes && capturing(ctx) &&
-        actq_layout(ActqRoute::rows, w->dtype, M, K, x).total <= ctx->ws_bytes)
+        actq_layout(ActqRoute::rows, w->dtype, M, N, K, x, c).total <= ctx->ws_bytes)
         return actq_run_within(ctx, w, row0, N, x, c, M, K, accumulate, static_cast<uint8_t *>(ctx->ws), ctx->ws_bytes, fast);
     uint8_t *ws = nullptr;
     if (l.total && !(ws = static_cast<uint8_t *>(workspace(ctx, l.total, &st)))) return st;
@@ -1217,10 +1223,10 @@ int trhip_gemm_q_actq_noalloc(trhip_ctx *ctx, const trhip_wstore *w, int64_t row
     const int r = actq_check(ctx, w, row0, N, x, c, M, K, "gemm_q_actq_noalloc", &st);
     if (r) return st;
     if (K != 0) {
-        ActqLayout l = actq_layout(actq_route(ctx, w->dtype, M, N, row0, K), w->dtype, M, K, x);
+        ActqLayout l = actq_layout(actq_route(ctx, w->dtype, M, N, row0, K), w->dtype, M, N, K, x, c);
         // tiles padded past the scratch: the row-major layout, which pads nothing, may still fit
         const bool within = l.total > (size_t)TRHIP_NOALLOC_SCRATCH_BYTES && l.route == ActqRoute::blocks;
-        if (within) l = actq_layout(ActqRoute::rows, w->dtype, M, K, x);
+        if (within) l = actq_layout(ActqRoute::rows, w->dtype, M, N, K, x, c);
         if (l.total > (size_t)TRHIP_NOALLOC_SCRATCH_BYTES)
             return fail(ctx, TRHIP_ERR_INVALID,
                         "gemm_q_actq_noalloc: M x K needs " + std::to_string(l.total) + " bytes of scratch; the static "

@@ -58,3 +58,20 @@ def test_actq_one_bad_row(backend, dt, bad):
     for b in (xb, cb):
         b.free()
     w.release()
+
+
+@pytest.mark.parametrize("dt", [Q4K, Q6K])
+@pytest.mark.parametrize("N,K,at", [(4096, 2048, 0), (9000, 4096, 1024), (1500, 4096, 3000)])
+def test_actq_token_over_its_input(backend, dt, N, K, at):
+    """One row whose outputs lie over its activations (from element `at` on): x is read before any of them is written."""
+    raw = O.small_scale_quant(dt, N, N * K // 256)
+    w = backend.FromQuantized(dt, raw, N, K)
+    x = np.random.default_rng(N).standard_normal(K).astype(np.float32)
+    want = O.quant_gemm_act(dt, 1, N, K, x.reshape(1, K), raw)
+    buf = backend.ctx.alloc((max(K, at + N) + 64) * 4)
+    for _ in range(4):
+        buf.upload(x)
+        backend.GemmActQuant(1, N, K, buf, w, (buf, at * 4), accumulate=False)
+        same_bits(buf.download(np.float32, N, byte_offset=at * 4), want)
+    buf.free()
+    w.release()
