@@ -97,3 +97,20 @@ def test_forced_plan_bits(backend, launch_shape, dt, plan, M, N, K):
     for b in (xb, cb, hb, hcb):
         b.free()
     w.release()
+
+
+@pytest.mark.parametrize("dt", [Q8, Q4, Q4K, Q6K])
+@pytest.mark.parametrize("M,N,K,at", [(3, 256, 256, 0), (20, 300, 512, 1000), (5, 70, 2304, 5000)])
+def test_rows_typed_over_its_input(backend, dt, M, N, K, at):
+    """c over x (from element `at` on): the call reads all of x, through its fp32 copy, before it writes c."""
+    raw = synth.quant_weights(dt, N, K, seed=N + K, outliers=0.01)
+    w = backend.FromQuantized(dt, raw, N, K)
+    h = O.round16(BF16, synth.activations(M, K, seed=K).reshape(-1))
+    want = O.widen16(BF16, O.round16(BF16, O.quant_gemm(dt, M, N, K, O.widen16(BF16, h).reshape(M, K), raw)))
+    buf = backend.ctx.alloc((max(M * K, at + M * N) + 64) * 2)
+    for _ in range(3):
+        buf.upload(h)
+        backend.GemmTyped(M, N, K, buf, BF16, w, (buf, 2 * at), BF16, accumulate=False, mode=MODE_EXACT)
+        same_bits(O.widen16(BF16, buf.download(np.uint16, M * N, byte_offset=2 * at)), want)
+    buf.free()
+    w.release()
