@@ -85,7 +85,8 @@ __device__ __forceinline__ int sdot4(uint32_t a, uint32_t b, int c) {
 }
 
 // One thread per output (m, n); blocks in order. Correct for every M: what the matrix-core kernels do not take (q4_0 of
-// few rows or a block count that is no multiple of 8; q4_k and q6_k whose padded tiles do not fit the static scratch).
+// few rows or a block count that is no multiple of 8; q4_k and q6_k where c lies over x and the padded tiles do not fit the
+// scratch; q4_k of fewer than 8 rows with a forced launch shape).
 template <int DT, bool ACC>
 __global__ __launch_bounds__(256) void actq_valu_kernel(const Planes p, int64_t N, int64_t row0, int64_t K,
                                                         const float *__restrict__ x, const int8_t *__restrict__ q,
@@ -226,8 +227,8 @@ int launch_quantize_q8(trhip_ctx *ctx, const float *x, int64_t M, int64_t K, int
     return launch_check(ctx, "quantize_q8");
 }
 
-// q4_k reaches this below actqw.hip's share only with a forced launch shape, or where its padded tiles do not fit the
-// static scratch.
+// (q4_k reaches this from 160 tiles of 64 x 128; below, only with a forced launch shape, or where c lies over x and the
+// padded tiles of actqw.hip do not fit the scratch)
 constexpr int64_t kActqMfmaMinRows = 8;
 
 int launch_actq_mfma(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c,

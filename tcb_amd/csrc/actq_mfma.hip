@@ -1056,8 +1056,9 @@ int launch_actq_mfma(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_
                      bool fast) {
     if (w->dtype != kQ4K) return fail(ctx, TRHIP_ERR_UNSUPPORTED, "actq_mfma: q4_k only");
     // Row-tile height: 64 rows unless that leaves fewer than 160 workgroups (measured: 4096 x 14336 at M = 128
-    // takes 74 us on 32-row tiles against 104 on 64; 14336 x 4096 at M = 128 or 512 is faster on 64).
-    // trhip_set_launch_shape(TRHIP_KNOB_ACTQ_TM) overrides.
+    // takes 74 us on 32-row tiles against 104 on 64; 14336 x 4096 at M = 128 or 512 is faster on 64). Such smaller grids
+    // run on actqw.hip; here only with forced K slices, or where the padding of its tiles does not fit the scratch and c
+    // lies over x. trhip_set_launch_shape(TRHIP_KNOB_ACTQ_TM) overrides.
     const int64_t wgs64 = ((N + TN - 1) / TN) * ((M + 63) / 64);
     const int tm = ctx->force_actq_tm ? ctx->force_actq_tm : (wgs64 < 160 ? 32 : 64);
     // K slices (fast mode): two when K is long (at least 32 blocks) and the tiles fit on the CUs one workgroup each.

@@ -1,6 +1,7 @@
 // actqw.hip -- act-quant product for q4_k and q6_k weights with the blocks of a row dealt over the waves of a
-// workgroup, bit-identical to dotQ4KQ8Go / dotQ6KQ8Go (tensor/cpu_quant_q8.go:91-116, 378-407). Taken wherever the
-// 128 x 256 tiles of prefill.hip would not fill the device: decode (M = 1) up to a few hundred rows.
+// workgroup, bit-identical to dotQ4KQ8Go / dotQ6KQ8Go (tensor/cpu_quant_q8.go:91-116, 378-407). Taken where the 128 x 256
+// tiles of prefill.hip would not fill the device, decode (M = 1) up to a few hundred rows; q4_k grids between the two, of
+// 160 tiles of 64 x 128 and more, stay on actq_mfma.hip (actq_blocks_applies).
 //
 // Per block b and output (m, n) the reference adds one fp32 value, blocks in order: acc = fl(acc + v_b) with
 //   q4_k: v_b = fl(fl(fl(d fl(isum)) - fl(dmin fl(msum))) d8)      q6_k: v_b = fl(fl(d fl(X)) d8)
@@ -118,11 +119,11 @@ __device__ __forceinline__ void expand_block(const uint8_t *img, int h, uint32_t
 // Activation operands of one 32-row tile and block in the tiled layout (trhip_internal.hpp): codes, the q4_k msum
 // operand and the scales of the lane's output rows. Lanes of rows past the tile's rows read row 0's (their outputs are
 // not stored; at M = 1 the other 31 rows would be 8 KB of padding per block).
-template <int DT, int RG>
+template <int DT>
 struct BlockA {
     v4i a[8];
     v8h s;
-    float4 d8[RG];
+    float4 d8[4];
     __device__ __forceinline__ void load(const int8_t *qt, const float *dt, const uint16_t *st, int64_t tb, int rows,
                                          int lane) {
         const int r = lane & 31, h = lane >> 5, l = r < rows ? lane : 32 * h;
@@ -132,18 +133,17 @@ struct BlockA {
         if (DT == kQ4K) s = *(reinterpret_cast<const v8h *>(st + tb * 512) + l);
         const float *dr = dt + tb * 32 + 4 * h;
 #pragma unroll
-        for (int q4 = 0; q4 < RG; q4++) d8[q4] = *reinterpret_cast<const float4 *>(dr + 8 * q4);
+        for (int q4 = 0; q4 < 4; q4++) d8[q4] = *reinterpret_cast<const float4 *>(dr + 8 * q4);
     }
 };
 
-// RG: of a tile's 32 rows only the first 8 RG are computed and exchanged (MT = 1, few rows). The value of output
-// (row 8 q + 4 h + i, column c) of tile t and wave w is component i of ex[w][(t 2 RG + 2 q + h) 32 + c]: one 16-byte
-// store per four outputs, whole 1 KB runs per wave, and the same for the reads of the sums.
-template <int DT, int MT, int RG, int W, int CW>
+// The value of output (row 8 q + 4 h + i, column c) of tile t and wave w is component i of ex[w][(8 t + 2 q + h) 32 + c]:
+// one 16-byte store per four outputs, whole 1 KB runs per wave, and the same for the reads of the sums.
+template <int DT, int MT, int W, int CW>
 struct Aw {
     static constexpr int BW = W / CW;                      // blocks a round
     static constexpr int TN = AW_TN * CW;                   // weight rows per workgroup
-    static constexpr int SLOTS = MT * RG * 64;              // float4 slots of a wave's tile
+    static constexpr int SLOTS = MT * 256;                  // float4 slots of a wave's tile
     // a wave's region, in float4: its block's images first, then (those read) its values
     static constexpr int REG = SLOTS * 16 > Raw<DT, 32>::BYTES ? SLOTS : Raw<DT, 32>::BYTES / 16;
     static constexpr int BUF = W * REG * 32 <= 131072 ? 2 : 1;  // two buffers (one barrier per round) where they fit
@@ -154,13 +154,13 @@ struct Aw {
 };
 
 // FAST (q4_k): the same integer sums, the two products of the epilogue fused (tolerance mode).
-template <int DT, int MT, int RG, int W, int CW, bool FAST>
+template <int DT, int MT, int W, int CW, bool FAST>
 __global__ __launch_bounds__(64 * W) void actq_blocks(const Planes p, int64_t N, int64_t row0, int64_t M, int64_t K,
                                                       const float *__restrict__ x, const int8_t *__restrict__ qt,
                                                       const float *__restrict__ dt, const uint16_t *__restrict__ st,
                                                       const uint8_t *__restrict__ bad_blk, float *__restrict__ c,
                                                       int acc) {
-    using T = Aw<DT, MT, RG, W, CW>;
+    using T = Aw<DT, MT, W, CW>;
     extern __shared__ __align__(16) uint8_t lds[];
     float4 *ex = reinterpret_cast<float4 *>(lds);
     int *rowstate = reinterpret_cast<int *>(lds + T::EX);  // [32 MT] 0 ok, 1 NaN/Inf row, 2 outside M
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(64 * W) void actq_blocks(const Planes p, int64_t N,
     // static; a guarded one makes the compiler wait for everything in flight, a memory latency per round.
     Raw<DT, 32> w0, w1;
     const int64_t nw = n0 + AW_TN * cw;  // this wave's first weight row
-    BlockA<DT, RG> A;
+    BlockA<DT> A;
     auto clamp_b = [&](int b) { return b < nb ? b : nb - 1; };
     w0.load(p, row0, nw, N, clamp_b(bw), lane);
     A.load(qt, dt, st, mt0 * nb + clamp_b(bw), mrows, lane);
@@ -214,15 +214,15 @@ __global__ __launch_bounds__(64 * W) void actq_blocks(const Planes p, int64_t N,
                     c0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(A.a[kc], lo[kc], c0, 0, 0, 0);
                     c1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(A.a[kc], hi[kc], c1, 0, 0, 0);
                 }
-                float4 d8[RG];
+                float4 d8[4];
 #pragma unroll
-                for (int q = 0; q < RG; q++) d8[q] = A.d8[q];
+                for (int q = 0; q < 4; q++) d8[q] = A.d8[q];
                 const bool last = t + 1 == MT || t + 1 == nt;  // the next round's first tile, or this one's next
                 const int64_t nx = last ? mt0 * nb + clamp_b(r0 + T::BW + bw) : (mt0 + t + 1) * nb + b;
                 A.load(qt, dt, st, nx, last ? mrows : mrows - 32 * (t + 1), lane);
                 if (t + 1 == MT) wn.load(p, row0, nw, N, clamp_b(r0 + T::AHEAD * T::BW + bw), lane);
 #pragma unroll
-                for (int q = 0; q < RG; q++) {
+                for (int q = 0; q < 4; q++) {
                     const float s8[4] = {d8[q].x, d8[q].y, d8[q].z, d8[q].w};
                     float v[4];
 #pragma unroll
@@ -234,7 +234,7 @@ __global__ __launch_bounds__(64 * W) void actq_blocks(const Planes p, int64_t N,
                         else tt = (dd * (float)(c0[e] + 8 * c1[e])) - (dm * cm[e]);
                         v[i] = tt * s8[i];
                     }
-                    xw[(t * 2 * RG + 2 * q + h) * 32 + r] = make_float4(v[0], v[1], v[2], v[3]);
+                    xw[(8 * t + 2 * q + h) * 32 + r] = make_float4(v[0], v[1], v[2], v[3]);
                 }
             } else if (t + 1 == MT) {
                 wn.load(p, row0, nw, N, clamp_b(r0 + T::AHEAD * T::BW + bw), lane);
@@ -276,7 +276,7 @@ __global__ __launch_bounds__(64 * W) void actq_blocks(const Planes p, int64_t N,
     for (int i = 0; i < T::OWN; i++) {
         const int s = tid + 64 * W * i;
         const int64_t gn = n0 + AW_TN * (s / T::SLOTS) + (s & 31);
-        const int ts = s % T::SLOTS, t = ts / (64 * RG), ml = 32 * t + 4 * ((ts >> 5) % (2 * RG));
+        const int ts = s % T::SLOTS, t = ts / 256, ml = 32 * t + 4 * ((ts >> 5) % 8);
         if (s < CW * T::SLOTS && t < nt && gn < N) {
             const float v[4] = {sum[i].x, sum[i].y, sum[i].z, sum[i].w};
 #pragma unroll
@@ -300,14 +300,14 @@ __global__ __launch_bounds__(64 * W) void actq_blocks(const Planes p, int64_t N,
     }
 }
 
-template <int DT, int MT, int RG, int W, int CW, bool FAST>
+template <int DT, int MT, int W, int CW, bool FAST>
 int go(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c, int64_t M, bool acc,
        const int8_t *qt, const float *dt, const uint16_t *st, const uint8_t *bad) {
-    using T = Aw<DT, MT, RG, W, CW>;
+    using T = Aw<DT, MT, W, CW>;
     static_assert(T::LDS <= 160 * 1024, "one workgroup per CU");
     const int64_t wgs = ((M + 32 * MT - 1) / (32 * MT)) * ((N + T::TN - 1) / T::TN);
     if (wgs >= ((int64_t)1 << 31)) return fail(ctx, TRHIP_ERR_UNSUPPORTED, "actq_blocks: grid too large");
-    const auto kern = &actq_blocks<DT, MT, RG, W, CW, FAST>;
+    const auto kern = &actq_blocks<DT, MT, W, CW, FAST>;
     const int s = allow_dyn_lds(ctx, reinterpret_cast<const void *>(kern), T::LDS, "actq_blocks: LDS size");
     if (s != TRHIP_OK) return s;
     hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(64 * W), T::LDS, ctx->stream, w->planes(), N, row0, M, w->K, x, qt,
@@ -619,16 +619,16 @@ int pick(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const f
         return TRHIP_AW(go_few, DT, (DT == kQ4K ? 2 : 1), 4, false);
     }
     if (M <= 32) {
-        if (!wide) return TRHIP_AW(go, DT, 1, 4, 8, 1);
-        return TRHIP_AW(go, DT, 1, 4, 8, 2);
+        if (!wide) return TRHIP_AW(go, DT, 1, 8, 1);
+        return TRHIP_AW(go, DT, 1, 8, 2);
     }
     // One workgroup fits a CU. While two-tile workgroups make one pass over the CUs they win (q4_k 128 rows, 4096 x
     // 14336: 37 us against 49 on three tiles); then three-tile ones while those do (130 rows: 50 against 59); beyond,
     // two column tiles per workgroup halve what each block's activations are read (256 rows: 63 against 66 and 87).
     const int64_t cols = (N + AW_TN - 1) / AW_TN;
-    if (cols * ((M + 63) / 64) <= cus) return TRHIP_AW(go, DT, 2, 4, 8, 1);
-    if (cols * ((M + 95) / 96) <= cus) return TRHIP_AW(go, DT, 3, 4, 8, 1);
-    return TRHIP_AW(go, DT, 2, 4, 8, 2);
+    if (cols * ((M + 63) / 64) <= cus) return TRHIP_AW(go, DT, 2, 8, 1);
+    if (cols * ((M + 95) / 96) <= cus) return TRHIP_AW(go, DT, 3, 8, 1);
+    return TRHIP_AW(go, DT, 2, 8, 2);
 #undef TRHIP_AW
 }
 
