@@ -689,57 +689,52 @@ namespace {
 struct Tiling {
     int wm;
     int64_t tiles, nch, nsl, cps;
+    double us;  // estimated
 };
-Tiling tiling(int64_t M, int64_t N, int64_t K, int64_t cus) {
+
+// Estimated time, fitted to measured ones (four formats, 256 to 128256 weight rows, K 256 to 14336, 17 to 2048 activation
+// rows, cold weights; within 7% rms).
+Tiling tiling_of(int wm, int dtype, int64_t M, int64_t N, int64_t K, int64_t cus) {
     Tiling t;
-    t.wm = M <= 32 ? 1 : M <= 64 ? 2 : 4;
-    t.tiles = ((M + 32 * t.wm - 1) / (32 * t.wm)) * ((N + FG_TN - 1) / FG_TN);
+    t.wm = wm;
+    t.tiles = ((M + 32 * wm - 1) / (32 * wm)) * ((N + FG_TN - 1) / FG_TN);
     t.nch = (K + 255) / 256;
     t.nsl = cus / t.tiles;
     if (t.nsl > t.nch / 2) t.nsl = t.nch / 2;
     if (t.nsl < 1) t.nsl = 1;
     t.cps = (t.nch + t.nsl - 1) / t.nsl;
     t.nsl = (t.nch + t.cps - 1) / t.cps;
+    static constexpr double chunk[4][3] = {{7.0, 8.6, 11.7}, {5.4, 7.0, 10.6}, {3.9, 4.9, 8.0}, {6.4, 8.5, 12.7}};
+    const double c = chunk[dtype == kQ8 ? 0 : dtype == kQ4 ? 1 : dtype == kQ4K ? 2 : 3][wm / 2];
+    const int64_t rounds = (t.tiles * t.nsl + cus - 1) / cus;
+    t.us = (double)rounds * (17.0 + (double)t.cps * c) + (double)(M * K) * 4e-6 / 3.0;
+    if (t.nsl > 1) t.us += 3.5 + (double)(t.nsl * M * N) * 8e-6 / 4.0;
     return t;
 }
-
-// Estimated times, us, fitted to measured ones (four formats, 256 to 128256 weight rows, K 256 to 14336, 17 to 2048
-// activation rows, cold weights; within 7% rms): this file's kernels, and the ones that q4_k and q6_k calls take otherwise
-// (actq_mfma.hip: 32- or 16-row tiles of 128 columns, two workgroups a CU, slices for 512 workgroups).
-double fast_gemm_time(int dtype, int64_t M, int64_t N, int64_t K, int64_t cus) {
-    const Tiling t = tiling(M, N, K, cus);
-    static constexpr double chunk[4][3] = {{7.0, 8.6, 11.1}, {5.4, 7.0, 10.4}, {3.9, 4.9, 8.0}, {6.4, 8.5, 12.7}};
-    const double c = chunk[dtype == kQ8 ? 0 : dtype == kQ4 ? 1 : dtype == kQ4K ? 2 : 3][t.wm / 2];
-    const int64_t rounds = (t.tiles * t.nsl + cus - 1) / cus;
-    const double us = (double)rounds * (17.0 + (double)t.cps * c) + (double)(M * K) * 4e-6 / 3.0;
-    return t.nsl > 1 ? us + 3.5 + (double)(t.nsl * M * N) * 8e-6 / 4.0 : us;
-}
-double small_tiles_time(int dtype, int64_t M, int64_t N, int64_t K, int64_t cus) {
-    const int64_t tm = dtype == kQ6K ? 16 : 32, nb = K / 256, tiles = ((N + 127) / 128) * ((M + tm - 1) / tm);
-    int64_t ns = (512 + tiles - 1) / tiles;
-    if (ns > nb) ns = nb;
-    const int64_t bps = (nb + ns - 1) / ns;
-    ns = (nb + bps - 1) / bps;
-    const double r = (double)(tiles * ns) / (double)(2 * cus), full = (double)((tiles * ns + 2 * cus - 1) / (2 * cus));
-    const double rounds = full <= 1.0 ? 1.0 : 0.7 * r + 0.3 * full;
-    const double us = 5.5 + rounds * (double)bps * (dtype == kQ6K ? 3.1 : 3.4) + (double)(M * K) * 4e-6 / 1.8 +
-                      (double)(M * N) * 1.1e-6;
-    return ns > 1 ? us + 2.5 + (double)(ns * M * N) * 8e-6 / 2.4 : us;
+Tiling tiling(int dtype, int64_t M, int64_t N, int64_t K, int64_t cus) {
+    const int wm = M <= 32 ? 1 : M <= 64 ? 2 : 4;
+    const Tiling t = tiling_of(wm, dtype, M, N, K, cus);
+    if (wm == 1) return t;
+    // half the height where that saves padded rows or fills the CUs (q4_k 20000 x 2048, 192 rows: 83 us in 128s, 60 in 64s)
+    const Tiling half = tiling_of(wm / 2, dtype, M, N, K, cus);
+    return half.us < 0.95 * t.us ? half : t;
 }
 
 }  // namespace
 
-// Where the two splitting launches and the 256-column tiles pay: by estimated time. q8_0 / q4_0, exact below (us, exact
+// Where the two splitting launches and the 256-column tiles pay. q8_0 / q4_0, exact below: by estimated time (us, exact
 // against this: 1024 x 4096, 64 rows q8_0 17, 38; 4096 x 4096, 64 rows 38, 41; 14336 x 4096, 32 rows 78, 54; 300 rows 575,
-// 185). q4_k, int8 digits below, from 7.5e9 multiply-adds, and q6_k, 16-row f16 tiles, from 4e9, except where the padding
-// to 128 rows takes more than it gives (20000 x 2048, 400 rows q4_k 160 here, 124 on digits; 129 rows q6_k 118, 88).
-// Rows below 256 elements stay exact: with so few sums the exact chain is nearer to float64 (K = 32: 4.9e-8 against 5.4e-8).
+// 195). q4_k, int8 digits below: from 7.5e9 multiply-adds (128 rows: 14336 x 4096 69, 68; 4096 x 4096 30, 44). q6_k,
+// 16-row f16 tiles below: from 4e9 (128 rows of 4096 x 4096 39, 52; 256 rows 59, 62). Past their lines a few shapes of the
+// k-quants would still be faster on the kernels below (20000 x 2048, 400 rows q4_k 157 here, 122), which are further from
+// float64 (4096 x 4096, 512 rows, x with a mean of 1, q4_k 1.5e-7 here, 1.1e-6). Rows below 256 elements stay exact: with
+// so few sums the exact chain is nearer to float64 (K = 32: 4.9e-8 against 5.4e-8).
 bool fast_gemm_pays(int dtype, int64_t M, int64_t N, int64_t K, int64_t cus) {
     if (M <= 16 || K < 256) return false;
-    const double macs = (double)M * (double)N * (double)K, t = fast_gemm_time(dtype, M, N, K, cus);
-    if (dtype == kQ4K || dtype == kQ6K)
-        return macs >= (dtype == kQ4K ? 7.5e9 : 4e9) && t < 1.03 * small_tiles_time(dtype, M, N, K, cus);
-    return t < 0.95 * gemm_rows_time(dtype, M, N, K, cus);
+    const double macs = (double)M * (double)N * (double)K;
+    if (dtype == kQ4K) return macs >= 7.5e9;
+    if (dtype == kQ6K) return macs >= 4e9;
+    return tiling(dtype, M, N, K, cus).us < 0.95 * gemm_rows_time(dtype, M, N, K, cus);
 }
 
 bool fast_gemm_applies(const trhip_ctx *ctx, int dtype, int64_t M, int64_t N, int64_t K) {
@@ -750,7 +745,7 @@ bool fast_gemm_applies(const trhip_ctx *ctx, int dtype, int64_t M, int64_t N, in
 int launch_fast_gemm(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x, float *c, int64_t M,
                      bool acc, float *swi) {
     const int64_t K = w->K, np = (K + 1023) / 1024, mt = (M + 31) / 32, KS = (K + 63) / 64 * 4;
-    const Tiling tl = tiling(M, N, K, ctx->sm_count > 0 ? ctx->sm_count : 256);
+    const Tiling tl = tiling(w->dtype, M, N, K, ctx->sm_count > 0 ? ctx->sm_count : 256);
     const int64_t nch = tl.nch, nsl = tl.nsl, cps = tl.cps;
     const int wm = tl.wm;
     auto al = [](size_t v) { return (v + 255) / 256 * 256; };

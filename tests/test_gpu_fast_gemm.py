@@ -46,7 +46,7 @@ def _row_errors(y, x, deq):
 
 # q8_0 / q4_0: 32-, 64- and 128-row tiles, ragged rows and columns, ragged 64-element steps, K slices; K below 256 (exact)
 SMALL = [(49, 33, 32, 0), (64, 257, 96, 3), (65, 256, 288, 0), (128, 300, 992, 1), (129, 255, 4096, 0), (50, 1030, 544, 2),
-         (17, 14500, 4096, 0), (33, 8000, 4096, 0)]
+         (17, 14500, 4096, 0), (33, 8000, 4096, 0), (300, 20000, 288, 0), (129, 11487, 2400, 1)]
 # k-quants: the smallest products that take this path
 # (and 17 to 32 rows, where only the widest stores do)
 LARGE = {Q4K: [(17, 700, 2304, 0), (32, 300, 4096, 3), (33, 513, 1024, 0), (129, 14336, 4096, 0), (460, 2051, 8192, 1), (64, 29000, 4096, 0), (2100, 14000, 256, 0)],
