@@ -715,9 +715,11 @@ Tiling tiling(int dtype, int64_t M, int64_t N, int64_t K, int64_t cus) {
     const int wm = M <= 32 ? 1 : M <= 64 ? 2 : 4;
     const Tiling t = tiling_of(wm, dtype, M, N, K, cus);
     if (wm == 1) return t;
-    // half the height where that saves padded rows or fills the CUs (q4_k 20000 x 2048, 192 rows: 83 us in 128s, 60 in 64s)
+    // half the height where that saves padded rows or fills the CUs (q4_k 20000 x 2048, 192 rows: 83 us in 128s, 66 in 64s)
+    // and leaves no fewer slices: longer sums round more (q8_0 10240 x 4096, 192 rows, two slices for three: error against
+    // float64 1.50e-7 for 1.43e-7)
     const Tiling half = tiling_of(wm / 2, dtype, M, N, K, cus);
-    return half.us < 0.95 * t.us ? half : t;
+    return half.us < 0.95 * t.us && half.cps <= t.cps ? half : t;
 }
 
 }  // namespace
