@@ -565,10 +565,11 @@ int run_dt(const RowsCall &r) {
 // (about two workgroups per CU in all) whose chain results are added in chunk order by sum_chunks_kernel.
 //
 // More rows: the plan of least estimated time, unless the walked one (16-row passes, one workgroup a row block and slice) is
-// within 6% of it. The costs below are fitted to 18 thousand measured times (four formats, 256 to 28672 rows, 17 to 1024
-// activation rows, cold weights): the plan taken is 1.1% over the best one in the mean, 15% at most, and over the walked
-// one at 1 of 1148 sizes by more than 3%. (Turns of one workgroup of kStageWaves or two of kSplitWaves a CU for every
-// format, in whole rounds, had put it over the walked plan by up to 32% at 76 of them: 4096 x 4096, M = 77, q8_0 55 -> 73.)
+// within 4% of it. The costs below are fitted to the measured times of every plan at 2948 sizes (four formats, 256 to 32768
+// rows, 17 to 2048 activation rows, cold weights): the plan taken is 1.2% over the best one in the mean, and over the
+// walked one by more than 3% at 10 of them, 10% at most. (Turns of one workgroup of kStageWaves or two of kSplitWaves a
+// CU for every format, in whole rounds of the device, had put it over the walked plan by up to 32%: 4096 x 4096, M = 77,
+// q8_0 55 -> 73 us.)
 //
 // A CU holds one workgroup of kStageWaves, and of kSplitWaves as many as their registers leave: two for q4_0 and q4_k, one
 // for q8_0 and q6_k (more than 256 registers a wave). Passes dealt over workgroups instead of walked by one fill the device
@@ -581,38 +582,44 @@ struct TurnCost {                        // us for a turn on 16 and on 32 activa
     double sums, l2_rate, rate;          // the partial sums' launch; MB / us of those that the L2s hold, of the rest
 };
 TurnCost turn_cost(int dtype) {
-    if (dtype == kQ8) return {{14.2, 25.1}, {7.7, 12.6}, {0, 0}, {6.8, 14.7}, 1.0, 1.2, 0.58, 0.7, 7.46, 4.6, 2.4};
-    if (dtype == kQ6K) return {{16.2, 29.0}, {9.1, 14.2}, {0, 0}, {6.0, 12.4}, 0.9, 0.9, 0.52, 0.58, 7.9, 4.0, 2.9};
-    return {{10.8, 18.4}, {5.9, 11.0}, {8.7, 16.2}, {3.9, 5.3}, 0.9, 0.9, 0.42, 0.68, 6.8, 5.8, 2.3};
+    if (dtype == kQ8) return {{14.2, 25.7}, {7.62, 13}, {0, 0}, {6.73, 17.7}, 1.4, 1.5, 0.71, 0.538, 6.68, 5.49, 2.03};
+    if (dtype == kQ6K) return {{16.2, 29.1}, {9.24, 14.8}, {0, 0}, {5.81, 12.6}, 0.884, 1.24, 0.729, 0.564, 6.71, 3.98, 2.37};
+    return {{10.8, 18.4}, {6.24, 10.1}, {8.66, 17.1}, {4.03, 5.21}, 0.857, 0.862, 0.334, 0.749, 6.89, 5.52, 2.3};
 }
 constexpr bool two_split_workgroups(int dtype) { return dtype == kQ4 || dtype == kQ4K; }
 
-// Passes one after another until the last of B workgroups for each of z ends, `slots` at a time in grid order: the first
-// np % z of the z take a pass more.
-int64_t passes_in_turn(int64_t B, int64_t np, int64_t z, int64_t slots) {
-    const int64_t q = np / z, heavy = np % z * B, f = heavy / slots, l = heavy % slots, rest = z * B - f * slots;
-    const int64_t t = f * (q + 1);
+// Workgroups are dealt in order over the shader engines (8 CUs each) and stay there, so that a plan lasts as long as the
+// engine with the most of them: 276 on 256 CUs leave one engine nine on eight CUs (q4_0 2944 x 1536, M = 343 in 32s: 73 us
+// in six workgroups a row block, 52 in eleven).
+constexpr int64_t kEngineCus = 8;
+
+// Passes one after another until the last of an engine's n workgroups ends, `slots` at a time in grid order; `heavy` of them,
+// the first, take q + 1 passes, the others q.
+int64_t passes_in_turn(int64_t n, int64_t heavy, int64_t q, int64_t slots) {
+    const int64_t f = heavy / slots, l = heavy % slots, rest = n - f * slots, t = f * (q + 1);
     if (rest <= 0) return t;
-    const int64_t n = (rest + slots - 1) / slots, last = rest - (n - 1) * slots;
-    if (l == 0) return t + n * q;
-    if (n == 1) return t + q + 1;
-    if (last > slots - l) return t + q + 1 + (n - 1) * q;
-    return t + (n * q > q + 1 + (n - 2) * q ? n * q : q + 1 + (n - 2) * q);
+    const int64_t r = (rest + slots - 1) / slots, last = rest - (r - 1) * slots;
+    if (l == 0) return t + r * q;
+    if (r == 1) return t + q + 1;
+    if (last > slots - l) return t + q + 1 + (r - 1) * q;
+    return t + (r * q > q + 1 + (r - 2) * q ? r * q : q + 1 + (r - 2) * q);
 }
 
 double plan_time(const RowsPlan &p, const TurnCost &cost, int dtype, int64_t M, int64_t N, int64_t nchunks, int64_t cus) {
     const bool cut = p.nslices > 1;
     const int64_t nrb = (N + 63) / 64, B = nrb * p.nslices, waves = cut ? kSplitWaves : kStageWaves;
     const int64_t np = (M + (p.two ? 31 : 15)) / (p.two ? 32 : 16), turns = (p.cps + waves - 1) / waves;
-    const bool pair = cut && two_split_workgroups(dtype) && B * p.pz > cus;
+    const int64_t engines = cus > kEngineCus ? cus / kEngineCus : 1, n = (B * p.pz + engines - 1) / engines;
+    const bool pair = cut && two_split_workgroups(dtype) && n > kEngineCus;
     // (up to kSplitWaves chunks leave a workgroup of kStageWaves one wave a SIMD)
     const double *turn = pair ? cost.pair : cut || nchunks <= kSplitWaves ? cost.alone : cost.whole;
-    const int64_t slots = pair ? 2 * cus : cus, rounds = (B * p.pz + slots - 1) / slots;
-    double t = (double)passes_in_turn(B, np, p.pz, slots) * ((double)turns * turn[p.two] + cost.pass);
+    const int64_t slots = pair ? 2 * kEngineCus : kEngineCus, rounds = (n + slots - 1) / slots;
+    const int64_t heavy = (np % p.pz * B + engines - 1) / engines, passes = passes_in_turn(n, heavy, np / p.pz, slots);
+    double t = (double)passes * ((double)turns * turn[p.two] + cost.pass);
     // (a start after the first overlaps the other workgroups' work in part)
     t += (1.0 + cost.later * (double)(rounds - 1)) * (cut ? cost.slice_start : cost.start[p.two]);
     // half a last pass: in every round where passes are walked, in its share of the rounds where each has its workgroup
-    const double halves = p.pz == 1 ? (double)rounds : p.pz == np ? (double)B / (double)slots : 0.0;
+    const double halves = p.pz == 1 ? (double)rounds : p.pz == np ? (double)B / (double)(slots * engines) : 0.0;
     if (p.two && M - 32 * (np - 1) <= 16) t -= cost.half * halves * (double)turns * (turn[1] - turn[0]);
     if (cut) {
         const double mb = (double)(nchunks * M * N) * 4e-6, l2 = mb < 32.0 ? mb : 32.0;
@@ -644,7 +651,7 @@ RowsPlan rows_plan(int dtype, int64_t M, int64_t N, int64_t nchunks, int64_t cus
     }
     const TurnCost cost = turn_cost(dtype);
     RowsPlan best = walked;
-    double least = 0.94 * plan_time(walked, cost, dtype, M, N, nchunks, cus);
+    double least = 0.96 * plan_time(walked, cost, dtype, M, N, nchunks, cus);
     for (int cut = 0; cut < (split.nslices > 1 ? 2 : 1); cut++)
         for (int two = 0; two < 2; two++) {
             RowsPlan p = cut ? split : whole;
@@ -667,11 +674,11 @@ RowsPlan rows_plan(int dtype, int64_t M, int64_t N, int64_t nchunks, int64_t cus
 
 }  // namespace
 
-// (the fitted costs rank plans; the time they give is 7% short for q8_0 and 15% for the others)
+// (the fitted costs rank plans; the time they give is 2% short for q8_0 and 15% for q4_0)
 double gemm_rows_time(int dtype, int64_t M, int64_t N, int64_t K, int64_t cus) {
     const int64_t nchunks = (K + 255) / 256;
     const RowsPlan p = rows_plan(dtype, M, N, nchunks, cus);
-    return plan_time(p, turn_cost(dtype), dtype, M, N, nchunks, cus) * (dtype == kQ8 ? 1.07 : 1.17);
+    return plan_time(p, turn_cost(dtype), dtype, M, N, nchunks, cus) * (dtype == kQ8 ? 1.02 : 1.15);
 }
 
 void gemm_rows_cut(int dtype, int64_t M, int64_t N, int64_t K, int64_t cus, int64_t plan[3]) {
