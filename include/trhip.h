@@ -93,9 +93,10 @@ int trhip_event_destroy(void *ev);
 /* Stream capture into a replayable HIP graph (launch-bound sequences such as a decode sweep).
  * Every call made on ctx between begin and end is recorded, not run; trhip_graph_launch replays it
  * on the context's stream. Calls that would grow the context's workspace fail during capture: make
- * one eager call of the same shapes first. A graph's nodes address the workspace as it was at
- * capture; when a later eager call grows it, the old buffers stay allocated until the context's last
- * graph is destroyed, so replays stay valid. Calls that wait for the stream, allocate or free
+ * one eager call of the same shapes first. (Products of more than 16 rows with 10177 weight rows and more, exact or
+ * q8_0 / q4_0 fast, and act-quant of q4_k and q6_k take a slower route instead that needs none or less.) A graph's
+ * nodes address the workspace as it was at capture; when a later eager call grows it, the old buffers stay allocated until
+ * the context's last graph is destroyed, so replays stay valid. Calls that wait for the stream, allocate or free
  * (trhip_sync, trhip_d2h, trhip_free, store creation and release, host-index embedding) refuse while
  * capturing. Counterpart of the reference's CUDA-graph replay (gpu/graph.go); nothing on this path
  * requires it. */
@@ -145,7 +146,8 @@ int trhip_wstore_to_raw(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int
  * block count), q4_k with 5 <= M <= 16 on f16 matrix cores over two-term activations and with M > 16
  * on int8 matrix cores, q4_0 with 2 <= M <= 16 (K a multiple of 256) and q6_k with M > 1 on f16 matrix
  * cores, and large products (M > 16) of every dtype on 16-bit matrix cores: q8_0 and q4_0 over three bf16
- * terms that hold x exactly, the k-quants over two f16 terms; other cases run exact. The reference GPU's GEMV and its
+ * terms that hold x exactly, the k-quants over two f16 terms (2^-23 of each element, and no less than 2^-39 of the
+ * largest of its row's 256-element block); other cases run exact. The reference GPU's GEMV and its
  * M > 1 dequantize-and-GEMM are tolerance-bound too (gpu/kernel_quant_gemv.go:33-84, gpu/backend_quant.go:43-134). */
 int trhip_gemm_q(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const float *x,
                  float *c, int64_t M, int64_t K, int accumulate, int mode);
@@ -156,8 +158,8 @@ int trhip_gemm_q(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N,
  * widened first when accumulating), and c is rounded to its type once, to nearest even (tensor/cpu_dtype.go:73-123:
  * NaN stays a quiet NaN, f16 overflows to Inf). Bit-identical to widening x, calling trhip_gemm_q and rounding its
  * result. With x and c of one 16-bit type (x 8-byte and c 2-byte aligned) the batch-1 GEMV (both modes) and the
- * fast batched decode read and write them directly; other cases go through fp32 copies in a workspace of the
- * context. */
+ * fast batched decode read and write them directly, as exact products of several rows do with 16-bit x and any c that
+ * does not lie over it; other cases go through fp32 copies in a workspace of the context. */
 int trhip_gemm_q_typed(trhip_ctx *ctx, const trhip_wstore *w, int64_t row0, int64_t N, const void *x, int xtype,
                        void *c, int ctype, int64_t M, int64_t K, int accumulate, int mode);
 
@@ -252,9 +254,9 @@ int trhip_rows_plan(int dtype, int64_t M, int64_t N, int64_t K, int cus, int64_t
  * (waves, K parts, rows in flight, rows per wave); TRHIP_KNOB_FAST_Q4K: row-sliced fast q4_k GEMV
  * (blocks in flight, waves, K parts, rows per lane); TRHIP_KNOB_EXACT_ROWS: exact four-lane GEMV rows
  * per workgroup a; TRHIP_KNOB_EXACT_LANES: exact GEMV lanes per row a (4, 8 or 16); TRHIP_KNOB_ACTQ_TM: act-quant
- * MFMA row tile a (0: built-in) and, in fast mode, b K slices (0: built-in); TRHIP_KNOB_ROWS16: fast q4_k kernel for 2..16 activation rows (a, b) = (16-row tiles per
- * wave 1 or 2; K slices 1..64, clamped to the block count); TRHIP_KNOB_KL_GRID: at least a workgroups for
- * the K-across-lanes fast GEMV (its rows dealt over more, shorter row groups); TRHIP_KNOB_ROWS: exact products of more
+ * MFMA row tile a (0: built-in) and, in fast mode, b K slices (0: built-in); TRHIP_KNOB_ROWS16: fast q4_k kernel for
+ * 2..16 activation rows (a, b) = (16-row tiles per wave 1 or 2; K slices 1..64, clamped to the block count);
+ * TRHIP_KNOB_KL_GRID: at least a workgroups for the K-across-lanes fast GEMV (its rows dealt over more, shorter row groups); TRHIP_KNOB_ROWS: exact products of more
  * than 16 activation rows (a, b, c) = (1: a row block's K chunks in one workgroup, 2: in slices where there are
  * enough of them; activation rows a pass, 16 or 32; workgroups its passes are dealt over); TRHIP_KNOB_FAST_GEMM: fast
  * mode of more than 16 rows, a = 1: always the f16 / bf16 matrix-core kernel (K of 256 up), 2: never. */

@@ -14,9 +14,10 @@
 // tiles: q6_k 4096 x 14336 at 130 rows ran 96 workgroups of 56 serial blocks, each wave expanding its weights for 64
 // activation rows only (366 us), and M = 1 ran a thread per output (q4_k 14336 x 4096 23 us). Here the grid is N / 32
 // tiles times 4 to 8 waves whatever K is, a weight block is expanded once for up to 96 activation rows, and the exchange
-// costs 8 KB of LDS traffic per 32 x 32 tile and block, beside 16 int8 MFMAs and about 100 VALU: 53 and 12.7 us. What
-// bounds it: VALU issue and the waits for it at two waves per SIMD (q6_k at 130 rows: 760 VALU per block, 440 of them
-// the expansion, VALU active 41% of the time, MFMA 17%); at M = 1 the start of each workgroup, then the weight bytes.
+// costs 8 KB of LDS traffic per 32 x 32 tile and block, beside 16 int8 MFMAs and about 100 VALU: 49.7 and 11.9 us. What
+// bounds it: VALU issue and the waits for it at two waves per SIMD (q6_k at 130 rows: 814 VALU per block, 440 of them the
+// expansion; of a SIMD's time VALU is active half, MFMA 19%: profiles/fast_gemm_and_actq_blocks.txt); at M = 1 the start of
+// each workgroup, then the weight bytes.
 #include "trhip_internal.hpp"
 #include "mfma_util.hpp"
 

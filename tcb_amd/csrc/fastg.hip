@@ -5,7 +5,7 @@
 // Activations: x is scaled by a power of two, x' = x 2^(14 - E), and split into terms.
 //   q8_0, q4_0: 2^E > max|x| of the row; three bf16 terms of eight bits, which add up to x' exactly, whatever the range of the row (bf16 has fp32's
 //     exponents; elements below 2^-110 of the row's largest lose low bits). Two f16 terms, exact to 2^-39 of the row's
-//     largest only, were 10-25% faster (4096 x 14336, M = 300 134 against 164 us) and lost every element beside one 2^40
+//     largest only, were 10-30% faster (4096 x 14336, M = 300 136 against 176 us) and lost every element beside one 2^40
 //     times larger.
 //   q4_k, q6_k: 2^E > max|x| of the row's 256-element block, which each block is multiplied back by where it is folded (one
 //     exponent a row loses the other blocks of a row that holds an outlier: a row of order 1 with one element of 1e8 was
@@ -16,8 +16,8 @@
 // so each product is exact and only fp32 sums round. Per block (32 elements for q8_0 and q4_0, 256 for the k-quants)
 //   acc += d D,   D = sum w x'   (over the terms);   q4_k: acc += d D + sum_j v_j S_j,   v_j = d o_j - dmin m_j
 // with S_j the sub-block sums of x' as three f16 terms and v_j, scaled by a power of two per block, as two. o_j is an
-// integer near dmin m_j / d, so that the code and minimum terms, several times the result, cancel in no sum. (Error
-// against float64 at K = 4096: 1.5e-7; with o_j = 8 sc_j 3.0e-7; the exact mode's 3.0e-7, the int8 digits' 2.2e-7.)
+// integer near dmin m_j / d, so that the code and minimum terms, several times the result, cancel in no sum. (q4_k, error
+// against float64 at K = 4096: 1.6e-7; with o_j = 8 sc_j 3.0e-7; the exact mode's 3.0e-7, the int8 digits' 2.2e-7.)
 //
 // Tiles. A workgroup is 8 waves over 32 WM activation rows and 256 weight rows. The weights of 64 elements are expanded
 // once per workgroup, by all threads, into LDS in operand order (two buffers, one barrier per 64 elements); a wave
@@ -25,12 +25,13 @@
 // each A operand, read straight from the split activations in L2, CT of them. (Weights expanded into each wave's own
 // registers would leave an A operand one MFMA at 32 columns a wave, and the A reads alone would fill the LDS bandwidth.)
 //
-// What bounds it: the matrix cores' rate under load and what is added to it. A plain f16 product reaches 1.38 PFLOP/s
-// here (24 ns per MFMA and SIMD, against 17 for int8), so the two products of 14336 x 4096 at M = 512 cannot take less
-// than 87 us; the kernel with its operand reads, expansion and folding taken out took 90, each of them adds its own time
-// (A reads 17 us, expansion 27, folding 12), whether the two waves of a SIMD work in step or in opposite phases: 144 us a
-// call (digits kernel 195). Multiplying before expanding, in each step, measured 143.8 against 152.6 us. q8_0 (exact
-// K = 1 products before): 14336 x 4096, M = 300 606 -> 185; 4096 x 14336, M = 300 725 -> 164.
+// What bounds it: the matrix cores' rate under load and what is added to it. A plain f16 product reaches 1.38 PFLOP/s here
+// (24 ns per MFMA and SIMD, against 17 for int8), so the two products of 14336 x 4096 at M = 512 (q4_k) cannot take less
+// than 87 us; beside its 2176 MFMAs a wave issues 9300 VALU, most of them the expansion and the fold (counters of both
+// kernels: profiles/fast_gemm_and_actq_blocks.txt). Operand reads, expansion and folding each added their own time when
+// put back one by one, whether the two waves of a SIMD worked in step or in opposite phases: 148 us a call (digits kernel
+// 196). Multiplying before expanding, in each step, measured 143.8 against 152.6 us (with one exponent a row). q8_0 (exact
+// K = 1 products before): 14336 x 4096, M = 300 606 -> 195; 4096 x 14336, M = 300 725 -> 176.
 #include "trhip_internal.hpp"
 #include "mfma_util.hpp"
 
