@@ -2,9 +2,9 @@
 // matrix cores: trhip_gemm_q(TRHIP_MODE_FAST). The reference's GPU runs these as dequantized tiles through a float GEMM
 // (gpu/backend_quant.go:43-134), a tolerance path too.
 //
-// Activations: x is scaled by a power of two, x' = x 2^(14 - E), and split into terms.
+// Activations: x is scaled by a power of two, x' = x 2^(80 - E) or x 2^(14 - E), and split into terms.
 //   q8_0, q4_0: 2^E > max|x| of the row; three bf16 terms of eight bits, which add up to x' exactly, whatever the range of the row (bf16 has fp32's
-//     exponents; elements below 2^-110 of the row's largest lose low bits). Two f16 terms, exact to 2^-39 of the row's
+//     exponents; elements below 2^-182 of the row's largest would lose low bits). Two f16 terms, exact to 2^-39 of the row's
 //     largest only, were 10-30% faster (4096 x 14336, M = 300 136 against 176 us) and lost every element beside one 2^40
 //     times larger.
 //   q4_k, q6_k: 2^E > max|x| of the row's 256-element block, which each block is multiplied back by where it is folded (one
@@ -44,12 +44,12 @@ typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef __bf16 v8b __attribute__((ext_vector_type(8)));
 
 constexpr int FG_W = 8, FG_THREADS = 64 * FG_W, FG_TN = 256;
-constexpr int FG_E = 14;  // |x'| < 2^14
 
 template <int DT>
 struct Fg {
     static constexpr bool KQ = DT == kQ4K || DT == kQ6K;
     static constexpr int TERMS = KQ ? 2 : 3;                  // of an activation
+    static constexpr int E = KQ ? 14 : 80;                    // |x'| < 2^E
     static constexpr int PL = DT == kQ6K ? 2 : 1;             // planes per weight
     static constexpr int B = PL * 4 * 8 * 1024;               // operands of a step: [plane][step][column tile][lane][16]
     static constexpr int DS = KQ ? 0 : 2 * FG_TN * 4;         // d of the step's two blocks
@@ -100,7 +100,8 @@ __global__ __launch_bounds__(256) void row_max_kernel(const float *__restrict__ 
 // in a dword). q8_0 / q4_0: three bf16 terms cut off x' in turn, eight bits each, so that they add up to x' exactly; a NaN
 // or Inf is its first term.
 // K is padded with zeros to a multiple of 64, rows to 32. q4_k: the sub-block sums S_j 2^-6 as three f16 terms, per tile
-// and 256-element block two operands [P0 | P1], [P0 | P2] (times [vh | vh], [vl | vh] of the weights). Workgroup (tile, 256-element chunk); ex[m] = E - 14, bad[m].
+// and 256-element block two operands [P0 | P1], [P0 | P2] (times [vh | vh], [vl | vh] of the weights). Workgroup (tile,
+// 256-element chunk); ex[m] = E of the row less Fg::E, bad[m], sx[tile][chunk][row] = 2^(the block's E - the row's).
 template <int DT>
 __global__ __launch_bounds__(256) void split_kernel(const float *__restrict__ x, int64_t M, int64_t K, int64_t np,
                                                     const float *__restrict__ pm, uint8_t *__restrict__ rec,
@@ -120,7 +121,7 @@ __global__ __launch_bounds__(256) void split_kernel(const float *__restrict__ x,
     int E = 0;
     if (!inf && a > 0.0f) (void)frexpf(a, &E);
     if (ch == 0 && s8 == 0 && row) {
-        ex[m] = E - FG_E;
+        ex[m] = E - Fg<DT>::E;
         if (Fg<DT>::KQ) bad[m] = inf ? 1 : 0;
     }
     const bool use = row && !inf;
@@ -162,7 +163,7 @@ __global__ __launch_bounds__(256) void split_kernel(const float *__restrict__ x,
         double s = 0.0;
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            v[i] = in ? ldexpf(raw[i], FG_E - E) : 0.0f;
+            v[i] = in ? ldexpf(raw[i], Fg<DT>::E - E) : 0.0f;
             if constexpr (TERMS == 3) {
                 const uint32_t u = __builtin_bit_cast(uint32_t, v[i]);
                 const bool fin = (u & 0x7F800000u) != 0x7F800000u;

@@ -153,9 +153,9 @@ def _outlier_case(dt, M, N, K, big):
 
 
 @pytest.mark.parametrize("dt,M,N", [(Q8, 130, 1024), (Q4, 130, 1024), (Q4K, 300, 6400), (Q6K, 300, 4096)])
-@pytest.mark.parametrize("big", [1e8, -1e20, 1e30])
+@pytest.mark.parametrize("big", [1e8, -1e20, 1e30, 3e38])
 def test_fast_gemm_outlier(backend, dt, M, N, big):
-    """The header's bound, |a - b| / (1 + |b|), unscaled, where one element is 1e8 to 1e30 times the others."""
+    """The header's bound, |a - b| / (1 + |b|), unscaled, where one element is 1e8 to 3e38 times the others."""
     K = 4096
     raw, x = _outlier_case(dt, M, N, K, big)
     w = backend.FromQuantized(dt, raw, N, K)
